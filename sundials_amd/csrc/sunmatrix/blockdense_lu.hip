@@ -7,24 +7,8 @@
 //   solver wrapper    src/sunlinsol/dense/sunlinsol_dense.c:128-183
 //   batched precedent src/sunlinsol/magmadense/sunlinsol_magmadense.cpp:314-440
 //
-// Kernel design (one m x m block per group of G = pow2ceil(m) lanes, 64/G
-// blocks per 64-wide wavefront, one wavefront per workgroup):
-//   * lane r holds row r of its block in registers (m values); every column
-//     load/store is one coalesced 8*m-byte segment per block;
-//   * partial pivoting without moving data: each lane carries the physical
-//     row position it currently occupies; the pivot search is a butterfly
-//     arg-max over the group keyed on (|a_rk|, -position), which reproduces
-//     the reference's "first maximum, strict >" choice in the reference's
-//     row order, and a "swap" just exchanges two position tags;
-//   * the pivot row is broadcast through LDS; each remaining row scales its
-//     multiplier with the reciprocal of the pivot and subtracts
-//     pivot_row[j] * multiplier column by column, skipping zero pivot-row
-//     entries -- the reference's exact per-element operation sequence, so in
-//     FP64 the factors are bit-identical;
-//   * rows are written back to their final physical position, so the stored
-//     factors and the pivot vector are those of the reference;
-//   * GETRS gathers b through the pivot sequence, then runs the unit-lower
-//     and upper sweeps with shuffle broadcasts of the solved entry.
+// The factorisation and solve kernels are in blocklu_device.h, compiled per
+// block size in the blocklu_inst_*.hip units.
 // The FP32 variant factors in single precision into a separate 4*m^2-byte
 // factor array and solves in FP64 arithmetic from those factors.
 // -----------------------------------------------------------------------------
@@ -35,10 +19,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <type_traits>
 
-#include "../core/lane_ops.h"
 #include "../core/profiler_internal.h"
+#include "blocklu.h"
 #include "sunamd/nvector_mi355.h"
 #include "sunamd/sunamd_profiler.h"
 #include "sunamd/sunmatrix_mi355block.h"
@@ -130,353 +113,8 @@ static int ew_grid(long n)
 }
 
 // ----------------------------------------------------------------------------
-// batched LU kernels
+// batched LU
 // ----------------------------------------------------------------------------
-__host__ __device__ constexpr int pow2ceil(int m)
-{
-  return m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : m <= 8 ? 8 : m <= 16 ? 16 : m <= 32 ? 32 : 64;
-}
-
-template <typename T>
-__device__ __forceinline__ T to_t(double v)
-{
-  return (T)v;
-}
-
-// How k_getrf forms the matrix it factors from its source blocks A:
-//   SRC_PLAIN  the blocks themselves;
-//   SRC_SCALED c*A + I (SUNMatScaleAddI's per-element a*c, then +1 on the
-//              diagonal), A read-only -- the Newton matrix from a saved
-//              Jacobian without the copy and the scaling pass;
-//   SRC_SAVE   as SRC_SCALED, and A's blocks are also written to `save` first
-//              (a fresh Jacobian kept for later setups).
-// With SRC_SCALED / SRC_SAVE and FP32 factors, `scaled` receives c*A + I in
-// FP64 -- the matrix the separate copy / scale / factor calls leave in the
-// solver's matrix; with FP64 factors the factors themselves go there.
-enum GetrfSource
-{
-  SRC_PLAIN  = 0,
-  SRC_SCALED = 1,
-  SRC_SAVE   = 2
-};
-
-// wavefronts per workgroup of the register-row factorisation (each wavefront
-// factors its own blocks; workgroups of several wavefronts put more blocks in
-// flight per CU than one-wavefront workgroups)
-#define LU_WAVES 4
-
-// Factor nblocks m x m blocks in place (T = double) or into an FP32 factor
-// array (T = float).  info receives min over failing blocks of
-// (block*m + k + 1) for the first zero pivot k.  Lane r of a block's group of
-// G = pow2ceil(m) lanes holds row r; the row swaps exchange position tags
-// only, and the rows are written to their final positions at the end.
-template <int M, typename T, int SRC = SRC_PLAIN>
-__global__ void __launch_bounds__(64 * LU_WAVES) k_getrf(const double* A, T* F /* may alias A */,
-                                                         int* __restrict__ piv, long nblocks,
-                                                         unsigned long long* info, double c = 0.0,
-                                                         double* save = nullptr,
-                                                         double* scaled = nullptr)
-{
-  using namespace sunamd_lane;
-  constexpr int G   = pow2ceil(M);
-  constexpr int BPW = 64 / G;
-  __shared__ T prow[LU_WAVES * BPW][M];
-
-  const int lane   = threadIdx.x & 63;
-  const int slot   = (threadIdx.x >> 6) * BPW + lane / G;
-  const int r      = lane % G;
-  const long blk   = (long)blockIdx.x * (LU_WAVES * BPW) + slot;
-  const bool valid = (blk < nblocks) && (r < M);
-
-  // every lane loads from inside block 0 or its own block (rows past M read
-  // row M-1), so the loads are unconditional and in flight together; idle
-  // lanes' values are replaced afterwards (a load under the validity test
-  // compiles to a branch per element, which waits for its load wherever a
-  // conversion or the scaling follows it).  FP32 factors, and the scaled
-  // forms at m > 32, take the FP64 source in chunks of 16 columns (a
-  // scheduling barrier between chunks), so the loads in flight do not cost the
-  // kernel its occupancy.
-  const long blk_s = (blk < nblocks) ? blk : 0;
-  const int r_s    = (r < M) ? r : M - 1;
-  const double* Ab = A + blk_s * (long)M * M;
-  const long o0    = blk * (long)M * M + r;
-  constexpr int CH = ((sizeof(T) == 4 && M > 16) || (SRC != SRC_PLAIN && M > 32)) ? 16 : M;
-  T a[M];
-#pragma unroll
-  for (int j0 = 0; j0 < M; j0 += CH)
-  {
-    double raw[CH];
-#pragma unroll
-    for (int q = 0; q < CH; q++)
-    {
-      if (j0 + q < M) { raw[q] = Ab[(j0 + q) * M + r_s]; }
-    }
-#pragma unroll
-    for (int q = 0; q < CH; q++)
-    {
-      const int j = j0 + q;
-      if (j >= M) { break; }
-      if (SRC == SRC_PLAIN) { a[j] = valid ? to_t<T>(raw[q]) : (T)0; }
-      else
-      {
-        double v = valid ? raw[q] : 0.0;
-        if (SRC == SRC_SAVE && valid) { save[o0 + (long)j * M] = v; }
-        v = v * c;
-        if (j == r) { v = v + 1.0; }
-        if (!std::is_same<T, double>::value && valid) { scaled[o0 + (long)j * M] = v; }
-        a[j] = valid ? to_t<T>(v) : (T)0;
-      }
-      // the single-precision value is formed here, not where it is first
-      // used (the compiler would otherwise keep the double until then)
-      if constexpr (sizeof(T) == 4) { asm volatile("" : "+v"(a[j])); }
-    }
-    if constexpr (CH < M) { __builtin_amdgcn_sched_barrier(0); }
-  }
-
-  int pos  = r; // physical row currently held by this lane
-  int myp  = 0; // pivot row chosen at step k == r
-  int fail = 0;
-
-#pragma unroll
-  for (int k = 0; k < M; k++)
-  {
-    // arg-max of |a_rk| over rows at positions >= k; ties -> lowest position
-    T v    = (valid && pos >= k) ? (T)fabs((double)a[k]) : (T)-1;
-    int bp = valid ? pos : INT_MAX;
-    g_argmax<G>(v, bp);
-    if (r == k) { myp = bp; }
-    if (v == (T)0 && fail == 0) { fail = k + 1; }
-
-    // exchange the position tags of rows k and bp
-    if (pos == k) { pos = bp; }
-    else if (pos == bp) { pos = k; }
-
-    const bool up = valid && pos > k && fail == 0;
-    if constexpr (G == 64)
-    {
-      // one block per wavefront: the pivot row's lane is wavefront-uniform,
-      // its entries are read straight from that lane's registers
-      const unsigned long long holder = __ballot(valid && pos == k);
-      const int pl = __builtin_amdgcn_readfirstlane(__ffsll((long long)holder) - 1) & 63;
-      const T pk   = readlane_d(a[k], pl);
-      T l          = (T)0;
-      if (up)
-      {
-        const T mult = (T)1 / pk;
-        l            = a[k] * mult;
-        a[k]         = l;
-      }
-#pragma unroll
-      for (int j = k + 1; j < M; j++)
-      {
-        const T pj = readlane_d(a[j], pl);
-        if (up && pj != (T)0) { a[j] = a[j] - pj * l; }
-      }
-    }
-    else
-    {
-      // the pivot row (now at position k) publishes columns k..M-1
-      wave_sync();
-      if (valid && pos == k)
-      {
-#pragma unroll
-        for (int j = k; j < M; j++) { prow[slot][j] = a[j]; }
-      }
-      wave_sync();
-      if (up)
-      {
-        const T mult = (T)1 / prow[slot][k];
-        const T l    = a[k] * mult;
-        a[k]         = l;
-#pragma unroll
-        for (int j = k + 1; j < M; j++)
-        {
-          const T pj = prow[slot][j];
-          if (pj != (T)0) { a[j] = a[j] - pj * l; }
-        }
-      }
-    }
-  }
-
-  if (valid)
-  {
-    T* Fb = F + blk * (long)M * M;
-#pragma unroll
-    for (int j = 0; j < M; j++) { Fb[j * M + pos] = a[j]; }
-    piv[blk * M + r] = myp;
-    if (r == 0 && fail != 0)
-    {
-      atomicMin(info, (unsigned long long)(blk * M + fail));
-    }
-  }
-}
-
-// x = LU^{-1} P b per block (x may alias b)
-template <int M, typename T>
-__global__ void __launch_bounds__(64) k_getrs(const T* __restrict__ F, const int* __restrict__ piv,
-                                              const double* b, double* x, long nblocks,
-                                              double scale = 1.0)
-{
-  constexpr int G   = pow2ceil(M);
-  constexpr int BPW = 64 / G;
-  const int lane    = threadIdx.x;
-  const int grp     = lane / G;
-  const int r       = lane % G;
-  const long blk    = (long)blockIdx.x * BPW + grp;
-  const bool valid  = (blk < nblocks) && (r < M);
-  const int base    = grp * G;
-
-  // every lane loads from inside block 0 or its own block (rows past M read
-  // row M-1), so the loads are unconditional and all in flight at once; the
-  // values of idle lanes are then replaced by zeros (a load under the
-  // validity test would be a branch per element, and for FP32 factors the
-  // conversion made each one wait for its load)
-  const long blk_s = (blk < nblocks) ? blk : 0;
-  const int r_s    = (r < M) ? r : M - 1;
-  const T* Fb      = F + blk_s * (long)M * M;
-  T raw[M];
-#pragma unroll
-  for (int j = 0; j < M; j++) { raw[j] = Fb[j * M + r_s]; }
-  const int* p = piv + blk_s * M;
-  int pv[M];
-#pragma unroll
-  for (int k = 0; k < M; k++) { pv[k] = p[k]; }
-  double lu[M];
-#pragma unroll
-  for (int j = 0; j < M; j++) { lu[j] = valid ? (double)raw[j] : 0.0; }
-
-  // source position of b after the sequential swaps b[k] <-> b[p[k]]
-  int idx = r_s;
-#pragma unroll
-  for (int k = M - 1; k >= 0; k--)
-  {
-    const int pk = pv[k];
-    if (idx == k) { idx = pk; }
-    else if (idx == pk) { idx = k; }
-  }
-  // (pivots of an unfactored block are not trusted to stay in range)
-  const double b_s = b[blk_s * M + (((unsigned)idx < (unsigned)M) ? idx : 0)];
-  double bi        = valid ? b_s : 0.0;
-
-  // L y = P b (unit lower)
-#pragma unroll
-  for (int k = 0; k < M - 1; k++)
-  {
-    double bk = __shfl(bi, base + k, 64);
-    if (r > k) { bi = bi - lu[k] * bk; }
-  }
-  // U x = y
-#pragma unroll
-  for (int k = M - 1; k > 0; k--)
-  {
-    if (r == k) { bi = bi / lu[k]; }
-    double bk = __shfl(bi, base + k, 64);
-    if (r < k) { bi = bi - lu[k] * bk; }
-  }
-  if (r == 0) { bi = bi / lu[0]; }
-  // scale * x is N_VScale's per-element product (exact for scale = 1)
-  if (valid) { x[blk * M + r] = scale * bi; }
-}
-
-// generic-size fallback (any m <= 64): block staged in LDS, same arithmetic
-template <typename T>
-__global__ void __launch_bounds__(64) k_getrf_lds(const double* A, T* F /* may alias A */,
-                                                  int* __restrict__ piv, long nblocks, int M,
-                                                  unsigned long long* info)
-{
-  extern __shared__ unsigned char smem_raw[];
-  T* s         = reinterpret_cast<T*>(smem_raw); // M*M, column-major, physical rows
-  const long blk = blockIdx.x;
-  const int r    = threadIdx.x;
-  if (blk >= nblocks) { return; }
-  const double* Ab = A + blk * (long)M * M;
-  for (int e = r; e < M * M; e += 64) { s[e] = to_t<T>(Ab[e]); }
-  __syncthreads();
-  __shared__ int sp[64];
-  __shared__ int sfail;
-  if (r == 0)
-  {
-    sfail = 0;
-    for (int k = 0; k < M; k++)
-    {
-      int l = k;
-      for (int i = k + 1; i < M; i++)
-      {
-        if (fabs((double)s[k * M + i]) > fabs((double)s[k * M + l])) { l = i; }
-      }
-      sp[k] = l;
-      if (s[k * M + l] == (T)0)
-      {
-        sfail = k + 1;
-        break;
-      }
-      if (l != k)
-      {
-        for (int j = 0; j < M; j++)
-        {
-          T t          = s[j * M + l];
-          s[j * M + l] = s[j * M + k];
-          s[j * M + k] = t;
-        }
-      }
-      T mult = (T)1 / s[k * M + k];
-      for (int i = k + 1; i < M; i++) { s[k * M + i] *= mult; }
-      for (int j = k + 1; j < M; j++)
-      {
-        T akj = s[j * M + k];
-        if (akj != (T)0)
-        {
-          for (int i = k + 1; i < M; i++) { s[j * M + i] = s[j * M + i] - akj * s[k * M + i]; }
-        }
-      }
-    }
-  }
-  __syncthreads();
-  T* Fb = F + blk * (long)M * M;
-  for (int e = r; e < M * M; e += 64) { Fb[e] = s[e]; }
-  if (r < M) { piv[blk * M + r] = sp[r]; }
-  if (r == 0 && sfail) { atomicMin(info, (unsigned long long)(blk * M + sfail)); }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(64) k_getrs_lds(const T* __restrict__ F, const int* __restrict__ piv,
-                                                  const double* b, double* x, long nblocks, int M)
-{
-  __shared__ double sb[64];
-  const long blk = blockIdx.x;
-  const int r    = threadIdx.x;
-  if (blk >= nblocks) { return; }
-  if (r < M) { sb[r] = b[blk * M + r]; }
-  __syncthreads();
-  if (r == 0)
-  {
-    const T* Fb  = F + blk * (long)M * M;
-    const int* p = piv + blk * M;
-    for (int k = 0; k < M; k++)
-    {
-      int pk = p[k];
-      if (pk != k)
-      {
-        double t = sb[k];
-        sb[k]    = sb[pk];
-        sb[pk]   = t;
-      }
-    }
-    for (int k = 0; k < M - 1; k++)
-    {
-      for (int i = k + 1; i < M; i++) { sb[i] = sb[i] - (double)Fb[k * M + i] * sb[k]; }
-    }
-    for (int k = M - 1; k > 0; k--)
-    {
-      sb[k] = sb[k] / (double)Fb[k * M + k];
-      for (int i = 0; i < k; i++) { sb[i] = sb[i] - (double)Fb[k * M + i] * sb[k]; }
-    }
-    sb[0] = sb[0] / (double)Fb[0];
-  }
-  __syncthreads();
-  if (r < M) { x[blk * M + r] = sb[r]; }
-}
-
 __global__ void k_info_reset(unsigned long long* info) { *info = ULLONG_MAX; }
 
 // ----------------------------------------------------------------------------
@@ -597,85 +235,54 @@ __global__ void __launch_bounds__(64) k_getrf_mfma(const double* __restrict__ A,
 // ----------------------------------------------------------------------------
 // launch dispatch over block sizes with register-resident kernels
 // ----------------------------------------------------------------------------
-#define LU_SIZES(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(12) X(16) X(24) X(32) X(48) X(64)
+// The launch tables.  Every size up to 64 has a register-row kernel: the
+// common ones with m constant, the others with m at run time in the next row
+// length of the second list.
+#define LU_EXACT_CASE(MM) case MM: return lu_size<MM, T>();
+#define LU_ROW_CASE(MM) if (m <= MM) { return lu_row_size<MM, T>(); }
+template <typename T>
+static const LuLaunch<T>* lu_launch(int m)
+{
+  switch (m)
+  {
+    LU_SIZES(LU_EXACT_CASE)
+  default: break;
+  }
+  LU_ROW_SIZES(LU_ROW_CASE)
+  return nullptr;
+}
 
 template <typename T>
 static bool launch_getrf(int m, const double* A, T* F, int* piv, long nblocks,
                          unsigned long long* info, hipStream_t s)
 {
-  switch (m)
-  {
-#define GETRF_CASE(MM)                                                                     \
-  case MM:                                                                                 \
-  {                                                                                        \
-    constexpr int BPG = LU_WAVES * (64 / pow2ceil(MM));                                    \
-    long g            = (nblocks + BPG - 1) / BPG;                                         \
-    k_getrf<MM, T><<<(unsigned)g, 64 * LU_WAVES, 0, s>>>(A, F, piv, nblocks, info);        \
-    return true;                                                                           \
-  }
-    LU_SIZES(GETRF_CASE)
-#undef GETRF_CASE
-  default: break;
-  }
-  if (m > 64) { return false; }
-  k_getrf_lds<T><<<(unsigned)nblocks, 64, sizeof(T) * m * m, s>>>(A, F, piv, nblocks, m, info);
+  const LuLaunch<T>* L = lu_launch<T>(m);
+  if (!L) { return false; }
+  L->getrf(m, A, F, piv, nblocks, info, s);
   return true;
 }
 
-// The register-resident sizes factor c*src + I in one pass (SRC_SCALED, or
-// SRC_SAVE with src also copied to save); false for other sizes, which take
+// The sizes compiled with m constant factor c*src + I in one pass (SRC_SCALED,
+// or SRC_SAVE with src also copied to save); false for other sizes, which take
 // the separate copy / scale / factor calls.
 template <typename T>
 static bool launch_getrf_scaled(int m, bool save_src, const double* src, double c, double* save,
                                 double* scaled, T* F, int* piv, long nblocks,
                                 unsigned long long* info, hipStream_t s)
 {
-  switch (m)
-  {
-#define GETRF_SC_CASE(MM)                                                                  \
-  case MM:                                                                                 \
-  {                                                                                        \
-    constexpr int BPG = LU_WAVES * (64 / pow2ceil(MM));                                    \
-    long g            = (nblocks + BPG - 1) / BPG;                                         \
-    if (save_src)                                                                          \
-    {                                                                                      \
-      k_getrf<MM, T, SRC_SAVE><<<(unsigned)g, 64 * LU_WAVES, 0, s>>>(                      \
-        src, F, piv, nblocks, info, c, save, scaled);                                      \
-    }                                                                                      \
-    else                                                                                   \
-    {                                                                                      \
-      k_getrf<MM, T, SRC_SCALED><<<(unsigned)g, 64 * LU_WAVES, 0, s>>>(                    \
-        src, F, piv, nblocks, info, c, save, scaled);                                      \
-    }                                                                                      \
-    return true;                                                                           \
-  }
-    LU_SIZES(GETRF_SC_CASE)
-#undef GETRF_SC_CASE
-  default: break;
-  }
-  return false;
+  const LuLaunch<T>* L = lu_launch<T>(m);
+  if (!L || !L->getrf_scaled) { return false; }
+  L->getrf_scaled(save_src, src, c, save, scaled, F, piv, nblocks, info, s);
+  return true;
 }
 
 template <typename T>
 static bool launch_getrs(int m, const T* F, const int* piv, const double* b, double* x,
                          long nblocks, hipStream_t s, double scale = 1.0)
 {
-  switch (m)
-  {
-#define GETRS_CASE(MM)                                                                     \
-  case MM:                                                                                 \
-  {                                                                                        \
-    constexpr int BPW = 64 / pow2ceil(MM);                                                 \
-    long g            = (nblocks + BPW - 1) / BPW;                                         \
-    k_getrs<MM, T><<<(unsigned)g, 64, 0, s>>>(F, piv, b, x, nblocks, scale);               \
-    return true;                                                                           \
-  }
-    LU_SIZES(GETRS_CASE)
-#undef GETRS_CASE
-  default: break;
-  }
-  if (m > 64 || scale != 1.0) { return false; }
-  k_getrs_lds<T><<<(unsigned)nblocks, 64, 0, s>>>(F, piv, b, x, nblocks, m);
+  const LuLaunch<T>* L = lu_launch<T>(m);
+  if (!L) { return false; }
+  L->getrs(m, F, piv, b, x, nblocks, scale, s);
   return true;
 }
 

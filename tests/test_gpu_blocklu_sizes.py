@@ -1,0 +1,114 @@
+"""Batched LU at every kind of block size: sizes compiled with m constant and
+sizes between them (m at run time in the next row length), around the lane
+groups' edges.  FP64 factors, pivots and solutions are the oracle's
+(oracle_block_getrf / _getrs) bit for bit; FP32 factors and pivots are those of
+the same algorithm in numpy float32, the solve from them in float64.  The
+blocks hold what the kernels treat apart: dense rows, rows full of zeros of
+both signs, tied pivots, a NaN, an infinity, and entries far outside the range
+of the reciprocal-based quotients."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from sundials_amd import _lib
+from helpers import dp, gpu_get, gpu_vec
+from test_gpu_blocklu import _gpu_matrix, _gpu_matrix_values, _to_blockmajor
+
+pytestmark = pytest.mark.gpu
+
+# both sides of every row length, and sizes with a kernel of their own
+SIZES = [2, 5, 9, 10, 11, 12, 13, 15, 16, 17, 20, 21, 23, 24, 25, 28, 29, 31, 32, 33, 40, 41, 47, 48,
+         49, 56, 57, 63, 64]
+
+
+def _cases(m, seed):
+    rng = np.random.default_rng(seed)
+    A = rng.uniform(-1, 1, (9, m, m))
+    A[1] *= rng.random((m, m)) < 0.3              # sparse, filling in
+    A[1] += np.diag(rng.uniform(1, 2, m))
+    A[2] = np.where(rng.random((m, m)) < 0.3, A[2], -0.0) + np.diag(rng.uniform(1, 2, m))
+    A[3] = np.sign(A[3]) + 2.0 * m * np.eye(m)[:, rng.permutation(m)]  # tied entries
+    A[4, :, 0] = 0.5                              # a tied column
+    A[5, m // 2, 0] = np.nan
+    A[6, m - 1, m - 1] = np.inf
+    A[7] = (np.eye(m) * 2.0 ** -900 if m % 2 else np.eye(m) * 2.0 ** 900)  # quotients by division
+    b = rng.uniform(-1, 1, (9, m))
+    b[8] *= rng.random(m) < 0.5
+    b[8, 0] = -0.0
+    return A, b
+
+
+def _numpy_getrf(A, T):
+    """SUNDlsMat_denseGETRF (sundials_dense.c:85-143) in precision T."""
+    a = A.astype(T)
+    m = len(a)
+    p = np.zeros(m, np.int64)
+    with np.errstate(all="ignore"):
+        for k in range(m):
+            l = k
+            for i in range(k + 1, m):
+                if abs(a[i, k]) > abs(a[l, k]):
+                    l = i
+            p[k] = l
+            if l != k:
+                a[[k, l]] = a[[l, k]]
+            a[k + 1:, k] *= T(1) / a[k, k]
+            for j in range(k + 1, m):
+                if a[k, j] != 0:
+                    a[k + 1:, j] -= a[k, j] * a[k + 1:, k]
+    return a, p
+
+
+def _solve(core, hip, ctx, A, b, prec):
+    nb, m, _ = A.shape
+    y = gpu_vec(ctx, np.zeros(nb * m))
+    M = _gpu_matrix(hip, ctx, y, A)
+    LS = hip.SUNLinSol_Mi355BlockLU(y, M, prec, ctx)
+    assert LS and core.SUNLinSolInitialize(LS) == 0
+    assert core.SUNLinSolSetup(LS, M) == 0
+    F = _gpu_matrix_values(hip, M, nb, m)
+    piv = np.zeros(nb * m, np.int32)
+    assert hip.SUNLinSol_Mi355BlockLU_GetPivots(LS, piv.ctypes.data_as(C.POINTER(C.c_int))) == 0
+    gb, gx = gpu_vec(ctx, b.ravel()), gpu_vec(ctx, np.zeros(nb * m))
+    assert core.SUNLinSolSolve(LS, M, gx, gb, 0.0) == 0
+    x = gpu_get(gx)
+    core.SUNLinSolFree(LS)
+    core.SUNMatDestroy(M)
+    for v in (y, gb, gx):
+        core.N_VDestroy(v)
+    return F, piv.reshape(nb, m), x.reshape(nb, m)
+
+
+@pytest.fixture
+def ctx():
+    c = _lib.new_context()
+    yield c
+    _lib.free_context(c)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("m", SIZES)
+def test_every_size_follows_the_dense_solver(ctx, m, prec):
+    core, hip, orc = _lib.core(), _lib.hip(), _lib.load_oracle()
+    A, b = _cases(m, 100 * m + prec)
+    if prec:
+        A = np.delete(A, 7, axis=0)  # 2^+-900 has no single-precision value
+        b = np.delete(b, 7, axis=0)
+    nb = len(A)
+    F, piv, x = _solve(core, hip, ctx, A, b, prec)
+    for k in range(nb):
+        a, p = _numpy_getrf(A[k], np.float32 if prec else np.float64)
+        finite = np.isfinite(A[k]).all()
+        assert np.array_equal(piv[k], p), ("pivots", k)
+        if prec == 0:
+            o = _to_blockmajor(A[k:k + 1]).copy()
+            q = np.zeros(m, np.int64)
+            assert orc.oracle_block_getrf(dp(o), m, q.ctypes.data_as(C.POINTER(C.c_int64))) == 0
+            assert np.array_equal(F[k * m * m:(k + 1) * m * m], o, equal_nan=True), ("factor", k)
+            assert np.array_equal(p, q)
+        # the solve in float64 from these factors, by the oracle
+        o = np.ascontiguousarray(a.T.astype(np.float64)).ravel()
+        r = b[k].copy()
+        orc.oracle_block_getrs(dp(o), m, p.ctypes.data_as(C.POINTER(C.c_int64)), dp(r))
+        assert np.array_equal(x[k], r, equal_nan=not finite), ("solve", k)
