@@ -12,10 +12,10 @@
 //    collapse to three per-element formulas, a*x+b*y, a*(x+y), a*(x-y)
 //    (nvector_serial.c:387-480 / :1600-1775), with no fused multiply-add;
 //  * reductions: per-lane sequential accumulation, 64-wide wavefront
-//    shuffle tree, LDS across wavefronts, per-workgroup partials; a
-//    one-workgroup finish kernel folds them in workgroup order and writes the
-//    scalar(s) straight into pinned host memory -- one stream synchronisation
-//    per reduction, deterministic results;
+//    shuffle tree, LDS across wavefronts, per-workgroup partials written
+//    straight into pinned host memory and folded there (up to 256 workgroups),
+//    or folded by a finish kernel that writes the scalar(s) there; the host
+//    watches the slots for the results -- deterministic, one round trip;
 //  * DotProdMulti reads x once for all nvec dot products (the serial vector
 //    re-reads x per product, nvector_serial.c:1019-1024) and spreads the work
 //    over the whole device (the reference uses one workgroup per product);
@@ -29,6 +29,8 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <ctime>
+#include <type_traits>
 
 #include "../core/profiler_internal.h"
 #include "sunamd/nvector_mi355.h"
@@ -38,12 +40,15 @@
 #define NV_MAX_MULTI 32      // vectors per fused call handled in one kernel
 #define NV_BLOCK 256         // threads per workgroup
 #define NV_MAX_RED_BLOCKS 2048
+#define NV_HOST_FOLD 256     // reductions of up to this many workgroups are folded on the host
 
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 
 // ----------------------------------------------------------------------------
 // execution context shared by a vector and all of its clones
 // ----------------------------------------------------------------------------
+#define NV_RESULT_SLOTS (NV_HOST_FOLD > NV_MAX_MULTI + 1 ? NV_HOST_FOLD : NV_MAX_MULTI + 1)
+
 struct Mi355Exec
 {
   int refcount;
@@ -51,10 +56,10 @@ struct Mi355Exec
   int num_cus;
   hipStream_t stream;
   double* d_partials;     // NV_MAX_RED_BLOCKS * (NV_MAX_MULTI + 1)
-  double* h_result;       // pinned, mapped: NV_MAX_MULTI + 1 scalars
+  double* h_result;       // pinned, mapped result slots (NV_RESULT_SLOTS)
   double* d_gs;           // Gram-Schmidt coefficients on the device (lazy, GS_MAX + 2)
-  double* h_gs;           // pinned copy of them (lazy)
   long int launches;
+  int watched;            // results taken from the slots since the last synchronisation
   hipError_t err;         // first HIP failure on this context since it was last read
   bool own_stream;
   bool is_default;
@@ -159,8 +164,8 @@ static Mi355Exec* exec_create(SUNContext ctx, hipStream_t user_stream, bool own_
                 sizeof(double) * NV_MAX_RED_BLOCKS * (NV_MAX_MULTI + 1));
   if (e == hipSuccess)
   {
-    e = hipHostMalloc((void**)&ex->h_result, sizeof(double) * (NV_MAX_MULTI + 1),
-                      hipHostMallocMapped);
+    e = hipHostMalloc((void**)&ex->h_result, sizeof(double) * NV_RESULT_SLOTS,
+                      hipHostMallocMapped | hipHostMallocCoherent);
   }
   if (e != hipSuccess)
   {
@@ -196,7 +201,6 @@ static void exec_release(Mi355Exec* ex)
   (void)hipFree(ex->d_partials);
   (void)hipHostFree(ex->h_result);
   if (ex->d_gs) { (void)hipFree(ex->d_gs); }
-  if (ex->h_gs) { (void)hipHostFree(ex->h_gs); }
   if (ex->own_stream) { (void)hipStreamDestroy(ex->stream); }
   if (ex->is_default && ex->device >= 0 && ex->device < 64 &&
       g_default_exec[ex->device] == ex)
@@ -213,10 +217,11 @@ static void exec_release(Mi355Exec* ex)
 // 128-bit loads per pair (measured sweeps over 6.3M-2^28 elements): 8 for one
 // or two input vectors (1 pair per lane per iteration leaves ~20 % of the
 // bandwidth unused), 4 for more -- at 2^28 a nine-vector dot product moves
-// 6.7 TB/s with 4 pairs per lane against 6.2-6.4 TB/s with 1.
+// 6.7 TB/s with 4 pairs per lane against 6.2-6.4 TB/s with 1 -- and 2 for more
+// than nine, whose loads in flight would not fit the registers otherwise.
 __host__ __device__ constexpr int unroll_for(int loads)
 {
-  return loads <= 2 ? 8 : 4;
+  return loads <= 2 ? 8 : (loads <= 9 ? 4 : 2);
 }
 
 // streaming: chunks of U * NV_BLOCK pairs per workgroup, grid capped at 32
@@ -229,6 +234,22 @@ static inline int stream_grid(const Mi355Exec* ex, sunindextype npairs, int U)
   if (g > cap) { g = cap; }
   if (g < 1) { g = 1; }
   return (int)g;
+}
+
+// Element pairs per lane of a streaming (elementwise) launch, which its result
+// does not depend on: U for vectors that give every CU four workgroups of
+// U-pair chunks, and fewer for shorter ones, whose few workgroups would leave
+// CUs idle (LinearSum of 32768 elements 2.8 -> 2.1 us, of 524288 4.85 ->
+// 4.5 us; at 2^25 8 pairs are the faster choice, see unroll_for).
+// launch(integral constant) is called with the choice.
+template <int LOADS, typename F>
+static inline void stream_launch(const Mi355Exec* ex, sunindextype npairs, F launch)
+{
+  constexpr int U                = unroll_for(LOADS);
+  const sunindextype full_grid   = 4 * (sunindextype)ex->num_cus;
+  if (npairs >= full_grid * U * NV_BLOCK) { launch(std::integral_constant<int, U>{}); }
+  else if (npairs >= full_grid * NV_BLOCK) { launch(std::integral_constant<int, 2>{}); }
+  else { launch(std::integral_constant<int, 1>{}); }
 }
 
 // The reduction grid depends only on the vector length and the kernel (not on
@@ -304,46 +325,49 @@ __device__ __forceinline__ void block_reduce(double (&v)[NV], double* lds /* NV*
   }
 }
 
-// Each workgroup publishes its NV partials; k_finish, launched next on the
-// same stream, folds them in workgroup order and writes the results to `out`
-// (pinned host memory or device memory).  Two launches instead of a
-// last-workgroup ticket: the kernel boundary orders the partials without a
-// device-scope fence and atomic per workgroup, which serialise at the end of
-// every reduction.
+// Each workgroup publishes its NV partials.  Up to NV_HOST_FOLD of them go
+// straight into the pinned result slots (one launch); more go to device memory
+// and k_finish, launched next on the same stream, folds them in workgroup
+// order into the slots.  No last-workgroup ticket: a device-scope fence and an
+// atomic per workgroup serialise at the end of every reduction.  A slot's
+// store is a system-scope atomic, so the host sees it before the kernel ends.
+__device__ __forceinline__ void store_result(double* p, double v)
+{
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <int OP, int NV>
-__device__ __forceinline__ void grid_finish(double (&v)[NV], double* partials)
+__device__ __forceinline__ void grid_finish(double (&v)[NV], double* partials, int to_host = 0)
 {
   __shared__ double lds[NV * (NV_BLOCK / 64)];
   block_reduce<OP, NV>(v, lds);
   if (threadIdx.x == 0)
   {
 #pragma unroll
-    for (int k = 0; k < NV; k++) { partials[k * gridDim.x + blockIdx.x] = v[k]; }
+    for (int k = 0; k < NV; k++)
+    {
+      double* p = &partials[k * gridDim.x + blockIdx.x];
+      if (to_host) { store_result(p, v[k]); }
+      else { *p = v[k]; }
+    }
   }
 }
 
-template <int OP, int NV>
+// workgroup k folds value k's partials (one workgroup over all values took
+// 19.5 us for 8 x 2048 partials, one each 5 us)
+template <int OP>
 __global__ void __launch_bounds__(NV_BLOCK) k_finish(const double* __restrict__ partials,
                                                      int nblocks, double* out, double identity)
 {
-  __shared__ double lds[NV * (NV_BLOCK / 64)];
-  double acc[NV];
-#pragma unroll
-  for (int k = 0; k < NV; k++)
+  __shared__ double lds[NV_BLOCK / 64];
+  const int k   = blockIdx.x;
+  double acc[1] = {identity};
+  for (int b = threadIdx.x; b < nblocks; b += NV_BLOCK)
   {
-    acc[k] = identity;
-    for (int b = threadIdx.x; b < nblocks; b += NV_BLOCK)
-    {
-      acc[k] = rcomb<OP>(acc[k], __builtin_nontemporal_load(&partials[k * nblocks + b]));
-    }
+    acc[0] = rcomb<OP>(acc[0], __builtin_nontemporal_load(&partials[k * nblocks + b]));
   }
-  block_reduce<OP, NV>(acc, lds);
-  if (threadIdx.x == 0)
-  {
-#pragma unroll
-    for (int k = 0; k < NV; k++) { out[k] = acc[k]; }
-    __threadfence_system();
-  }
+  block_reduce<OP, 1>(acc, lds);
+  if (threadIdx.x == 0) { store_result(&out[k], acc[0]); }
 }
 
 // ----------------------------------------------------------------------------
@@ -393,13 +417,13 @@ enum LSMode
   LS_SCALEDIF = 2  // a*(x-y)
 };
 
-template <int MODE>
+template <int MODE, int U>
 __global__ void __launch_bounds__(NV_BLOCK) k_linearsum(double a, const double* __restrict__ x,
                                                         double b, const double* __restrict__ y,
                                                         double* __restrict__ z, long n)
 {
   const long np = n >> 1;
-  chunk_pairs<unroll_for(2)>(
+  chunk_pairs<U>(
     np, [&](long i) { return Pairs<2>{{ld2(x, i), ld2(y, i)}}; },
     [&](long i, const Pairs<2>& p) {
       dbl2 r;
@@ -450,7 +474,7 @@ __device__ __forceinline__ double ew(double x, double y, double c)
   return (fabs(x) >= c) ? 1.0 : 0.0;
 }
 
-template <int OP>
+template <int OP, int U>
 __global__ void __launch_bounds__(NV_BLOCK) k_ew(const double* __restrict__ x,
                                                  const double* __restrict__ y, double c,
                                                  double* __restrict__ z, long n)
@@ -458,7 +482,7 @@ __global__ void __launch_bounds__(NV_BLOCK) k_ew(const double* __restrict__ x,
   const bool binary = (OP == EW_PROD || OP == EW_DIV);
   const long np     = n >> 1;
   constexpr int NL  = binary ? 2 : 1;
-  chunk_pairs<unroll_for(NL)>(
+  chunk_pairs<U>(
     np,
     [&](long i) {
       Pairs<NL> p;
@@ -551,7 +575,8 @@ template <int K>
 __global__ void __launch_bounds__(NV_BLOCK) k_reduce(const double* __restrict__ x,
                                                      const double* __restrict__ y,
                                                      const double* __restrict__ id, long n,
-                                                     double identity, double* partials)
+                                                     double identity, double* partials,
+                                                     int to_host)
 {
   const int OP     = RedTraits<K>::op;
   const bool two   = (K == RK_DOT || K == RK_WSQR || K == RK_WSQRMASK);
@@ -580,7 +605,7 @@ __global__ void __launch_bounds__(NV_BLOCK) k_reduce(const double* __restrict__ 
     acc[0] = rcomb<OP>(acc[0], red_elem<K>(x[n - 1], two ? y[n - 1] : 0.0,
                                           three ? id[n - 1] : 0.0));
   }
-  grid_finish<OP, 1>(acc, partials);
+  grid_finish<OP, 1>(acc, partials, to_host);
 }
 
 // Left-to-right sums in the serial vector's order (nvector_serial.c:605-761):
@@ -612,7 +637,7 @@ __global__ void __launch_bounds__(64) k_reduce_seq(const double* __restrict__ x,
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) { out[0] = acc; }
+  if (threadIdx.x == 0) { store_result(out, acc); }
 }
 
 // fused d_k = x . Y_k, k < NV (x read once)
@@ -687,11 +712,11 @@ __global__ void __launch_bounds__(NV_BLOCK) k_dotmulti(const double* __restrict_
 
 // z = c0*X0; z += c_k*X_k (k = 1..nvec-1): the rounding of the generic-layer
 // loop (sundials_nvector.c:549-572), one pass, z written once
-template <int NV>
+template <int NV, int U>
 __global__ void __launch_bounds__(NV_BLOCK) k_lincomb(CoefPack c, PtrPack X, double* z, long n)
 {
   const long np = n >> 1;
-  chunk_pairs<unroll_for(NV)>(
+  chunk_pairs<U>(
     np,
     [&](long i) {
       Pairs<NV> p;
@@ -715,12 +740,12 @@ __global__ void __launch_bounds__(NV_BLOCK) k_lincomb(CoefPack c, PtrPack X, dou
 }
 
 // Z_k = a_k*x + Y_k (k < NV); x read once
-template <int NV>
+template <int NV, int U>
 __global__ void __launch_bounds__(NV_BLOCK) k_scaleaddmulti(CoefPack a, const double* __restrict__ x,
                                                             PtrPack Y, WPtrPack Z, long n)
 {
   const long np = n >> 1;
-  chunk_pairs<unroll_for(NV + 1)>(
+  chunk_pairs<U>(
     np,
     [&](long i) {
       Pairs<NV + 1> p;
@@ -741,11 +766,11 @@ __global__ void __launch_bounds__(NV_BLOCK) k_scaleaddmulti(CoefPack a, const do
 }
 
 // Z_k = c_k * X_k (k < NV)
-template <int NV>
+template <int NV, int U>
 __global__ void __launch_bounds__(NV_BLOCK) k_scalearray(CoefPack c, PtrPack X, WPtrPack Z, long n)
 {
   const long np = n >> 1;
-  chunk_pairs<unroll_for(NV)>(
+  chunk_pairs<U>(
     np,
     [&](long i) {
       Pairs<NV> p;
@@ -861,20 +886,15 @@ static void mi_linearsum(sunrealtype a, N_Vector x, sunrealtype b, N_Vector y, N
   long n = (long)NVLEN(z);
   if (n == 0) { return; }
   Mi355Exec* ex = EXEC(z);
-  int g         = stream_grid(ex, n >> 1, unroll_for(2));
   sunamd_prof_begin(SUNAMD_K_LINSUM, ex->stream);
-  if (a == b)
-  {
-    k_linearsum<LS_SCALESUM><<<g, NV_BLOCK, 0, ex->stream>>>(a, DDATA(x), b, DDATA(y), DDATA(z), n);
-  }
-  else if (a == -b)
-  {
-    k_linearsum<LS_SCALEDIF><<<g, NV_BLOCK, 0, ex->stream>>>(a, DDATA(x), b, DDATA(y), DDATA(z), n);
-  }
-  else
-  {
-    k_linearsum<LS_GENERIC><<<g, NV_BLOCK, 0, ex->stream>>>(a, DDATA(x), b, DDATA(y), DDATA(z), n);
-  }
+  stream_launch<2>(ex, n >> 1, [&](auto uc) {
+    constexpr int U = decltype(uc)::value;
+    const int g     = stream_grid(ex, n >> 1, U);
+    auto kern       = (a == b)    ? k_linearsum<LS_SCALESUM, U>
+                      : (a == -b) ? k_linearsum<LS_SCALEDIF, U>
+                                  : k_linearsum<LS_GENERIC, U>;
+    kern<<<g, NV_BLOCK, 0, ex->stream>>>(a, DDATA(x), b, DDATA(y), DDATA(z), n);
+  });
   sunamd_prof_end(SUNAMD_K_LINSUM, ex->stream);
   LAUNCHCHK(z);
 }
@@ -917,9 +937,12 @@ static void mi_ew(N_Vector x, N_Vector y, double c, N_Vector z)
   long n = (long)NVLEN(z);
   if (n == 0) { return; }
   Mi355Exec* ex = EXEC(z);
-  const int nl = (OP == EW_PROD || OP == EW_DIV) ? 2 : 1;
-  k_ew<OP><<<stream_grid(ex, n >> 1, unroll_for(nl)), NV_BLOCK, 0, ex->stream>>>(
-    DDATA(x), y ? DDATA(y) : DDATA(x), c, DDATA(z), n);
+  constexpr int nl = (OP == EW_PROD || OP == EW_DIV) ? 2 : 1;
+  stream_launch<nl>(ex, n >> 1, [&](auto uc) {
+    constexpr int U = decltype(uc)::value;
+    k_ew<OP, U><<<stream_grid(ex, n >> 1, U), NV_BLOCK, 0, ex->stream>>>(
+      DDATA(x), y ? DDATA(y) : DDATA(x), c, DDATA(z), n);
+  });
   LAUNCHCHK(z);
 }
 
@@ -944,6 +967,78 @@ static void mi_compare(sunrealtype c, N_Vector x, N_Vector z)
   mi_ew<EW_COMPARE>(x, NULL, c, z);
 }
 
+// ---- results from the device ------------------------------------------------
+// A result slot is set to this value (a NaN of a pattern that no arithmetic
+// produces) before the launch that fills it, and the host watches it change: a
+// reduction's answer is then there about as soon as its last store, where a
+// stream synchronisation adds its own wake-up.  A slot that does not change
+// within SLOT_WAIT_S -- a kernel that takes longer, an error, a launch inside a
+// stream capture -- is left to hipStreamSynchronize, which also reports the
+// error.  Everything earlier on the stream is complete when the slot changes.
+static constexpr unsigned long long SLOT_EMPTY = 0x7ff4a3d5c2e1b709ULL;
+static constexpr double SLOT_WAIT_S            = 2e-3;
+// Every so many results the stream is synchronised all the same: the runtime
+// retires finished launches there, and a backlog of them (thousands, after
+// some hundred steps) would be retired at the caller's next synchronising call
+// instead.  It costs each result 1/SLOT_SYNC_EVERY of a synchronisation.
+static constexpr int SLOT_SYNC_EVERY = 32;
+
+static inline void slots_clear(Mi355Exec* ex, int count)
+{
+  volatile unsigned long long* p = (volatile unsigned long long*)ex->h_result;
+  for (int i = 0; i < count; i++) { p[i] = SLOT_EMPTY; }
+  __atomic_thread_fence(__ATOMIC_RELEASE);
+}
+
+static hipError_t slots_wait(Mi355Exec* ex, int count)
+{
+  volatile unsigned long long* p = (volatile unsigned long long*)ex->h_result;
+  struct timespec t0, t;
+  bool timed = false;
+  for (int i = 0; i < count; i++)
+  {
+    for (long spins = 0; p[i] == SLOT_EMPTY; spins++)
+    {
+      if ((spins & 255) == 255)
+      {
+        clock_gettime(CLOCK_MONOTONIC, timed ? &t : &t0);
+        if (timed && (double)(t.tv_sec - t0.tv_sec) + 1e-9 * (double)(t.tv_nsec - t0.tv_nsec) > SLOT_WAIT_S)
+        {
+          return hipStreamSynchronize(ex->stream);
+        }
+        timed = true;
+      }
+    }
+  }
+  __atomic_thread_fence(__ATOMIC_ACQUIRE);
+  if (++ex->watched < SLOT_SYNC_EVERY) { return hipSuccess; }
+  ex->watched = 0;
+  return hipStreamSynchronize(ex->stream);
+}
+
+// k_finish's order for up to NV_HOST_FOLD (= one per thread) partials: the
+// wavefronts' trees, then the wavefronts in order
+template <int OP>
+static double fold_on_host(const double* p, int n, double identity)
+{
+  static_assert(NV_HOST_FOLD <= NV_BLOCK, "one partial per thread of k_finish");
+  auto comb = [](double a, double b) {
+    return OP == RSUM ? a + b : OP == RMAX ? (b > a ? b : a) : (b < a ? b : a);
+  };
+  double r = identity;
+  for (int w = 0; w < NV_BLOCK / 64; w++)
+  {
+    double v[64];
+    for (int l = 0; l < 64; l++) { v[l] = (64 * w + l < n) ? comb(identity, p[64 * w + l]) : identity; }
+    for (int off = 32; off >= 1; off >>= 1)
+    {
+      for (int l = 0; l < off; l++) { v[l] = comb(v[l], v[l + off]); }
+    }
+    r = (w == 0) ? v[0] : comb(r, v[0]);
+  }
+  return r;
+}
+
 // run one reduction kernel, wait for it, return the host-visible result
 template <int K>
 static double mi_reduce(N_Vector x, N_Vector y, N_Vector id, double identity)
@@ -954,7 +1049,11 @@ static double mi_reduce(N_Vector x, N_Vector y, N_Vector id, double identity)
   int g = red_grid(ex, n >> 1, unroll_for(red_loads<K>()));
   const int fam = (K == RK_WSQR) ? SUNAMD_K_WRMS : -1;
   // min / max are exact in any order; sums follow the vector's reduction order
-  const bool seq = (RedTraits<K>::op == RSUM) && CONTENT(x)->red_order == SUNAMD_REDUCE_SEQUENTIAL;
+  constexpr int OP = RedTraits<K>::op;
+  const bool seq   = (OP == RSUM) && CONTENT(x)->red_order == SUNAMD_REDUCE_SEQUENTIAL;
+  const bool fold  = !seq && g <= NV_HOST_FOLD;
+  const int slots  = fold ? g : 1;
+  slots_clear(ex, slots);
   if (fam >= 0) { sunamd_prof_begin(fam, ex->stream); }
   if (seq)
   {
@@ -965,14 +1064,17 @@ static double mi_reduce(N_Vector x, N_Vector y, N_Vector id, double identity)
   {
     k_reduce<K><<<g, NV_BLOCK, 0, ex->stream>>>(DDATA(x), y ? DDATA(y) : DDATA(x),
                                                 id ? DDATA(id) : DDATA(x), n, identity,
-                                                ex->d_partials);
-    k_finish<RedTraits<K>::op, 1><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g,
-                                                                 ex->h_result, identity);
+                                                fold ? ex->h_result : ex->d_partials, fold);
+    if (!fold)
+    {
+      k_finish<OP><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->h_result, identity);
+    }
   }
   if (fam >= 0) { sunamd_prof_end(fam, ex->stream); }
   LAUNCHCHK(x);
-  HIPCHK_EX(x, hipStreamSynchronize(ex->stream));
-  return (ex->err == hipSuccess) ? ex->h_result[0] : NAN;
+  HIPCHK_EX(x, slots_wait(ex, slots));
+  if (ex->err != hipSuccess) { return NAN; }
+  return fold ? fold_on_host<OP>(ex->h_result, g, identity) : ex->h_result[0];
 }
 
 static sunrealtype mi_dotprod(N_Vector x, N_Vector y) { return mi_reduce<RK_DOT>(x, y, NULL, 0.0); }
@@ -1002,7 +1104,7 @@ static sunbooleantype mi_invtest(N_Vector x, N_Vector z)
   if (n == 0) { return SUNTRUE; }
   const int g = red_grid(ex, n >> 1, 4);
   k_invtest<<<g, NV_BLOCK, 0, ex->stream>>>(DDATA(x), DDATA(z), n, ex->d_partials);
-  k_finish<RMAX, 1><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->h_result, 0.0);
+  k_finish<RMAX><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->h_result, 0.0);
   LAUNCHCHK(x);
   HIPCHK(x->sunctx, hipStreamSynchronize(ex->stream));
   return (ex->h_result[0] > 0.0) ? SUNFALSE : SUNTRUE;
@@ -1015,7 +1117,7 @@ static sunbooleantype mi_constrmask(N_Vector c, N_Vector x, N_Vector m)
   if (n == 0) { return SUNTRUE; }
   const int g = red_grid(ex, n >> 1, 4);
   k_constrmask<<<g, NV_BLOCK, 0, ex->stream>>>(DDATA(c), DDATA(x), DDATA(m), n, ex->d_partials);
-  k_finish<RMAX, 1><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->h_result, 0.0);
+  k_finish<RMAX><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->h_result, 0.0);
   LAUNCHCHK(x);
   HIPCHK(x->sunctx, hipStreamSynchronize(ex->stream));
   return (ex->h_result[0] > 0.0) ? SUNFALSE : SUNTRUE;
@@ -1028,7 +1130,7 @@ static sunrealtype mi_minquotient(N_Vector num, N_Vector den)
   if (n == 0) { return SUN_BIG_REAL; }
   const int g = red_grid(ex, n >> 1, 4);
   k_minquotient<<<g, NV_BLOCK, 0, ex->stream>>>(DDATA(num), DDATA(den), n, ex->d_partials);
-  k_finish<RMIN, 1><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->h_result, DBL_MAX);
+  k_finish<RMIN><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->h_result, DBL_MAX);
   LAUNCHCHK(num);
   HIPCHK(num->sunctx, hipStreamSynchronize(ex->stream));
   return ex->h_result[0];
@@ -1037,6 +1139,9 @@ static sunrealtype mi_minquotient(N_Vector num, N_Vector den)
 // ---- fused ops --------------------------------------------------------------
 #define NV_CASES(MACRO) \
   MACRO(1) MACRO(2) MACRO(3) MACRO(4) MACRO(5) MACRO(6) MACRO(7) MACRO(8)
+// kernels that take up to NV_WIDE vectors in one pass
+#define NV_WIDE 12
+#define NV_WIDE_CASES(MACRO) NV_CASES(MACRO) MACRO(9) MACRO(10) MACRO(11) MACRO(12)
 
 static SUNErrCode mi_dotprodmulti(int nvec, N_Vector x, N_Vector* Y, sunrealtype* d)
 {
@@ -1072,6 +1177,7 @@ static SUNErrCode mi_dotprodmulti(int nvec, N_Vector x, N_Vector* Y, sunrealtype
     for (int k = 0; k < nv; k++) { P.p[k] = DDATA(Y[base + k]); }
     double* slot = ex->h_result + (base - group);
     int g        = 0;
+    if (base == group) { slots_clear(ex, nvec - group < NV_MAX_MULTI ? nvec - group : NV_MAX_MULTI); }
     sunamd_prof_begin(SUNAMD_K_DOTMULTI, ex->stream);
     switch (nv)
     {
@@ -1079,7 +1185,7 @@ static SUNErrCode mi_dotprodmulti(int nvec, N_Vector x, N_Vector* Y, sunrealtype
   case NVV:                                                                                \
     g = red_grid(ex, n >> 1, unroll_for(NVV + 1));                                         \
     k_dotmulti<NVV><<<g, NV_BLOCK, 0, ex->stream>>>(DDATA(x), P, n, ex->d_partials);       \
-    k_finish<RSUM, NVV><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, slot, 0.0);     \
+    k_finish<RSUM><<<NVV, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, slot, 0.0);        \
     break;
       NV_CASES(DM_CASE)
 #undef DM_CASE
@@ -1089,7 +1195,7 @@ static SUNErrCode mi_dotprodmulti(int nvec, N_Vector x, N_Vector* Y, sunrealtype
     int filled = base + nv - group;
     if (filled == NV_MAX_MULTI || base + nv == nvec)
     {
-      HIPCHK_EX(x, hipStreamSynchronize(ex->stream));
+      HIPCHK_EX(x, slots_wait(ex, filled));
       for (int k = 0; k < filled; k++) { d[group + k] = ex->h_result[k]; }
       group += filled;
     }
@@ -1113,7 +1219,7 @@ static SUNErrCode mi_lincomb(int nvec, sunrealtype* c, N_Vector* X, N_Vector z)
     int nv;
     if (done == 0)
     {
-      nv = nvec < 8 ? nvec : 8;
+      nv = nvec < NV_WIDE ? nvec : NV_WIDE;
       for (int k = 0; k < nv; k++)
       {
         C.c[k] = c[k];
@@ -1122,7 +1228,7 @@ static SUNErrCode mi_lincomb(int nvec, sunrealtype* c, N_Vector* X, N_Vector z)
     }
     else
     {
-      nv     = (nvec - done) + 1 < 8 ? (nvec - done) + 1 : 8;
+      nv     = (nvec - done) + 1 < NV_WIDE ? (nvec - done) + 1 : NV_WIDE;
       C.c[0] = 1.0;
       P.p[0] = DDATA(z);
       for (int k = 1; k < nv; k++)
@@ -1135,10 +1241,13 @@ static SUNErrCode mi_lincomb(int nvec, sunrealtype* c, N_Vector* X, N_Vector z)
     {
 #define LC_CASE(NVV)                                                                    \
   case NVV:                                                                             \
-    k_lincomb<NVV><<<stream_grid(ex, n >> 1, unroll_for(NVV)), NV_BLOCK, 0, ex->stream>>>( \
-      C, P, DDATA(z), n);                                                                 \
+    stream_launch<NVV>(ex, n >> 1, [&](auto uc) {                                       \
+      constexpr int U = decltype(uc)::value;                                            \
+      k_lincomb<NVV, U><<<stream_grid(ex, n >> 1, U), NV_BLOCK, 0, ex->stream>>>(       \
+        C, P, DDATA(z), n);                                                             \
+    });                                                                                 \
     break;
-      NV_CASES(LC_CASE)
+      NV_WIDE_CASES(LC_CASE)
 #undef LC_CASE
     }
     LAUNCHCHK(z);
@@ -1170,8 +1279,11 @@ static SUNErrCode mi_scaleaddmulti(int nvec, sunrealtype* a, N_Vector x, N_Vecto
     {
 #define SAM_CASE(NVV)                                                                        \
   case NVV:                                                                                  \
-    k_scaleaddmulti<NVV><<<stream_grid(ex, n >> 1, unroll_for(NVV + 1)), NV_BLOCK, 0,           \
-                           ex->stream>>>(C, DDATA(x), P, W, n);                                \
+    stream_launch<NVV + 1>(ex, n >> 1, [&](auto uc) {                                        \
+      constexpr int U = decltype(uc)::value;                                                 \
+      k_scaleaddmulti<NVV, U><<<stream_grid(ex, n >> 1, U), NV_BLOCK, 0, ex->stream>>>(      \
+        C, DDATA(x), P, W, n);                                                               \
+    });                                                                                      \
     break;
       NV_CASES(SAM_CASE)
 #undef SAM_CASE
@@ -1203,8 +1315,11 @@ static SUNErrCode mi_scalevectorarray(int nvec, sunrealtype* c, N_Vector* X, N_V
     {
 #define SVA_CASE(NVV)                                                                  \
   case NVV:                                                                            \
-    k_scalearray<NVV><<<stream_grid(ex, n >> 1, unroll_for(NVV)), NV_BLOCK, 0,            \
-                        ex->stream>>>(C, P, W, n);                                       \
+    stream_launch<NVV>(ex, n >> 1, [&](auto uc) {                                      \
+      constexpr int U = decltype(uc)::value;                                           \
+      k_scalearray<NVV, U><<<stream_grid(ex, n >> 1, U), NV_BLOCK, 0, ex->stream>>>(   \
+        C, P, W, n);                                                                   \
+    });                                                                                \
     break;
       NV_CASES(SVA_CASE)
 #undef SVA_CASE
@@ -1643,19 +1758,34 @@ __global__ void __launch_bounds__(NV_BLOCK) k_gs_update(double* vk, PtrPack V,
   if (last) { grid_finish<RSUM, 1>(nrm, partials); }
 }
 
+// the new norm^2 (folded as k_finish folds it) and the ncoef coefficients into
+// the result slots, coefficients first
+__global__ void __launch_bounds__(NV_BLOCK) k_finish_gs(const double* __restrict__ partials,
+                                                        int nblocks, const double* __restrict__ d,
+                                                        int ncoef, double* out)
+{
+  __shared__ double lds[NV_BLOCK / 64];
+  if ((int)threadIdx.x < ncoef) { store_result(&out[threadIdx.x], d[threadIdx.x]); }
+  double acc[1] = {0.0};
+  for (int b = threadIdx.x; b < nblocks; b += NV_BLOCK)
+  {
+    acc[0] = rcomb<RSUM>(acc[0], __builtin_nontemporal_load(&partials[b]));
+  }
+  block_reduce<RSUM, 1>(acc, lds);
+  if (threadIdx.x == 0) { store_result(&out[ncoef], acc[0]); }
+}
+static_assert(GS_MAX + 2 <= NV_RESULT_SLOTS && GS_MAX + 1 <= NV_BLOCK, "k_finish_gs's slots");
+
+// vectors per pass when `count` of them go in the fewest passes of equal width
+static int gs_width(int count)
+{
+  const int passes = (count + NV_WIDE - 1) / NV_WIDE;
+  return (count + passes - 1) / passes;
+}
+
 static bool gs_buffers(Mi355Exec* ex)
 {
-  if (ex->d_gs && ex->h_gs) { return true; }
-  if (!ex->d_gs && hipMalloc((void**)&ex->d_gs, sizeof(double) * (GS_MAX + 2)) != hipSuccess)
-  {
-    return false;
-  }
-  if (!ex->h_gs && hipHostMalloc((void**)&ex->h_gs, sizeof(double) * (GS_MAX + 2),
-                                 hipHostMallocDefault) != hipSuccess)
-  {
-    return false;
-  }
-  return true;
+  return ex->d_gs || hipMalloc((void**)&ex->d_gs, sizeof(double) * (GS_MAX + 2)) == hipSuccess;
 }
 
 // Same arguments, coefficients and reorthogonalisation rule as SUNClassicalGS;
@@ -1678,10 +1808,12 @@ extern "C" SUNErrCode SUNAMD_ClassicalGS_Mi355(N_Vector* v, sunrealtype** h, int
   {
     return SUNClassicalGS(v, h, k, p, new_vk_norm, stemp, vtemp);
   }
-  // projections d_j = v_k . v_(i0+j), j < nv, and v_k . v_k into d_gs[0..nv]
-  for (int base = 0; base <= nv; base += 8)
+  // projections d_j = v_k . v_(i0+j), j < nv, and v_k . v_k into d_gs[0..nv],
+  // in as few passes over v_k as NV_WIDE allows, of equal width
+  const int wide = gs_width(nv + 1);
+  for (int base = 0; base <= nv; base += wide)
   {
-    int cnt = nv + 1 - base < 8 ? nv + 1 - base : 8;
+    int cnt = nv + 1 - base < wide ? nv + 1 - base : wide;
     PtrPack P;
     for (int j = 0; j < cnt; j++) { P.p[j] = DDATA(v[i0 + base + j]); }
     int g = 0;
@@ -1691,20 +1823,22 @@ extern "C" SUNErrCode SUNAMD_ClassicalGS_Mi355(N_Vector* v, sunrealtype** h, int
   case NVV:                                                                                 \
     g = red_grid(ex, n >> 1, unroll_for(NVV + 1));                                          \
     k_dotmulti<NVV><<<g, NV_BLOCK, 0, ex->stream>>>(DDATA(vk), P, n, ex->d_partials);       \
-    k_finish<RSUM, NVV><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->d_gs + base,  \
-                                                        0.0);                               \
+    k_finish<RSUM><<<NVV, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->d_gs + base,     \
+                                                     0.0);                                   \
     break;
-      NV_CASES(GD_CASE)
+      NV_WIDE_CASES(GD_CASE)
 #undef GD_CASE
     }
     LAUNCHCHK(vk);
   }
   // v_k -= sum_j d_j v_j (the reference's linear combination pairs the
-  // coefficient of v_(i0+j) with v[j]; identical when i0 == 0), new norm^2
-  // into d_gs[nv + 1]
-  for (int base = 0; base < nv; base += 8)
+  // coefficient of v_(i0+j) with v[j]; identical when i0 == 0); the new norm^2
+  // joins the coefficients in the result slots
+  const int uwide = gs_width(nv);
+  slots_clear(ex, nv + 2);
+  for (int base = 0; base < nv; base += uwide)
   {
-    int cnt  = nv - base < 8 ? nv - base : 8;
+    int cnt  = nv - base < uwide ? nv - base : uwide;
     int last = (base + cnt == nv) ? 1 : 0;
     PtrPack P;
     for (int j = 0; j < cnt; j++) { P.p[j] = DDATA(v[base + j]); }
@@ -1718,20 +1852,18 @@ extern "C" SUNErrCode SUNAMD_ClassicalGS_Mi355(N_Vector* v, sunrealtype** h, int
                                                      ex->d_partials);                        \
     if (last)                                                                                \
     {                                                                                        \
-      k_finish<RSUM, 1><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->d_gs + nv + 1, \
-                                                        0.0);                                \
+      k_finish_gs<<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->d_gs, nv + 1,       \
+                                                  ex->h_result);                             \
     }                                                                                        \
     break;
-      NV_CASES(GU_CASE)
+      NV_WIDE_CASES(GU_CASE)
 #undef GU_CASE
     }
     LAUNCHCHK(vk);
   }
-  HIPCHK_EX(vk, hipMemcpyAsync(ex->h_gs, ex->d_gs, sizeof(double) * (nv + 2),
-                               hipMemcpyDeviceToHost, ex->stream));
-  HIPCHK_EX(vk, hipStreamSynchronize(ex->stream));
+  HIPCHK_EX(vk, slots_wait(ex, nv + 2));
   if (ex->err != hipSuccess) { return SUN_ERR_EXT_FAIL; }
-  const double* d      = ex->h_gs;
+  const double* d      = ex->h_result;
   const double vk_norm = (d[nv] <= 0.0) ? 0.0 : sqrt(d[nv]);
   for (int i = 0; i < nv; i++) { h[i][k_minus_1] = d[i]; }
   *new_vk_norm = (d[nv + 1] <= 0.0) ? 0.0 : sqrt(d[nv + 1]);

@@ -1,0 +1,109 @@
+"""Vector ops at the lengths where their launches change: one to several
+element pairs per lane (streaming ops), reductions folded on the host up to
+256 workgroups and by the finish kernel beyond, Gram-Schmidt steps of one and
+more passes of up to 12 vectors, and a reduction that outlasts the host's
+watch on its result slot.  Elementwise results equal numpy's float64 bit for
+bit; a sum of n terms in any order is within n * 2^-53 * sum |terms| of the
+exact one (twice that here: the products round too)."""
+import ctypes as C
+import math
+
+import numpy as np
+import pytest
+
+from sundials_amd import _lib
+from helpers import dp, gpu_get, gpu_vec, vec_array
+
+pytestmark = pytest.mark.gpu
+
+# 256 and 257 workgroups of 4096 (one or two inputs) and of 2048 elements
+# (three); the streaming thresholds 2 * 4 * 256 * 256 and that times 8 elements
+EDGES = [1, 2, 4095, 4097, 524287, 524288, 524290, 526337, 1048576, 1048577, 1052673, 4194303, 4194306]
+
+
+@pytest.fixture
+def ctx():
+    c = _lib.new_context()
+    yield c
+    _lib.free_context(c)
+
+
+def _close(got, terms):
+    exact = math.fsum(terms)
+    return abs(got - exact) <= 2 * len(terms) * 2.0 ** -53 * math.fsum(np.abs(terms)) + 0.0
+
+
+@pytest.mark.parametrize("n", EDGES)
+def test_launch_edges(ctx, n):
+    core = _lib.core()
+    rng = np.random.default_rng(n)
+    x, y, w = rng.standard_normal(n), rng.standard_normal(n), rng.uniform(0.5, 2, n)
+    vx, vy, vw, vz = (gpu_vec(ctx, a) for a in (x, y, w, np.zeros(n)))
+    idv = np.where(rng.random(n) < 0.7, 1.0, 0.0)
+    vi = gpu_vec(ctx, idv)
+    core.N_VLinearSum(0.3, vx, -0.7, vy, vz)
+    assert np.array_equal(gpu_get(vz), 0.3 * x + (-0.7) * y)
+    core.N_VScale(-2.5, vx, vz)
+    assert np.array_equal(gpu_get(vz), -2.5 * x)
+    core.N_VDiv(vx, vw, vz)
+    assert np.array_equal(gpu_get(vz), x / w)
+    c = (C.c_double * 3)(0.5, -1.25, 3.0)
+    assert core.N_VLinearCombination(3, c, vec_array([vx, vy, vw]), vz) == 0
+    assert np.array_equal(gpu_get(vz), (0.5 * x + -1.25 * y) + 3.0 * w)
+    assert _close(core.N_VDotProd(vx, vy), x * y)
+    assert _close(core.N_VL1Norm(vx), np.abs(x))
+    assert core.N_VMaxNorm(vx) == np.abs(x).max() and core.N_VMin(vx) == x.min()
+    for got, terms in ((core.N_VWrmsNorm(vx, vw), (x * w) ** 2),
+                       (core.N_VWrmsNormMask(vx, vw, vi), (x * w) ** 2 * idv)):
+        assert _close(got * got * n, terms) or abs(got * got * n / math.fsum(terms) - 1) <= (2 * n + 4) * 2.0 ** -53
+    d = (C.c_double * 3)()
+    assert core.N_VDotProdMulti(3, vx, vec_array([vx, vy, vw]), d) == 0
+    assert all(_close(d[k], x * t) for k, t in enumerate((x, y, w)))
+    # what is not finite comes through a result slot like any value
+    x[n // 2] = np.nan
+    vn = gpu_vec(ctx, x)
+    assert math.isnan(core.N_VDotProd(vn, vy))
+    x[n // 2] = np.inf
+    vf = gpu_vec(ctx, x)
+    assert core.N_VL1Norm(vf) == math.inf and core.N_VMaxNorm(vf) == math.inf
+    for v in (vx, vy, vw, vz, vi, vn, vf):
+        core.N_VDestroy(v)
+
+
+def test_reduction_longer_than_the_watch(ctx):
+    """Sequential order: one lane adds four million terms, far longer than the
+    host watches the slot before it synchronises."""
+    core, hip = _lib.core(), _lib.hip()
+    n = 4000001
+    x = np.random.default_rng(3).standard_normal(n)
+    v = gpu_vec(ctx, x)
+    assert hip.N_VSetReductionOrder_Mi355(v, 1) == 0
+    want = np.cumsum(np.abs(x))[-1]  # left to right
+    for _ in range(2):
+        assert core.N_VL1Norm(v) == want
+    core.N_VDestroy(v)
+
+
+@pytest.mark.parametrize("k", [1, 8, 11, 12, 13, 23, 24, 25, 30])
+def test_gram_schmidt_passes(ctx, k):
+    core, hip = _lib.core(), _lib.hip()
+    n = 70001
+    rng = np.random.default_rng(k)
+    q = np.linalg.qr(rng.standard_normal((n, k)))[0].T.copy()
+    w = rng.standard_normal(n)
+    vs = [gpu_vec(ctx, a) for a in q] + [gpu_vec(ctx, w)]
+    tmp = [gpu_vec(ctx, np.zeros(n)) for _ in range(k + 1)]
+    h = np.zeros((k + 1, k))
+    PD = C.POINTER(C.c_double)
+    rows = (PD * (k + 1))(*[C.cast(h[i].ctypes.data, PD) for i in range(k + 1)])
+    norm, stemp = C.c_double(), (C.c_double * (k + 2))()
+    assert hip.SUNAMD_ClassicalGS_Mi355(vec_array(vs), rows, k, k, C.byref(norm), stemp,
+                                        vec_array(tmp)) == 0
+    assert all(_close(h[i, k - 1], q[i] * w) for i in range(k))
+    z = w.copy()
+    for i in range(k):
+        z = z + -h[i, k - 1] * q[i]
+    assert np.array_equal(gpu_get(vs[-1]), z)
+    assert abs(norm.value / np.linalg.norm(z) - 1) <= n * 2.0 ** -53
+    for v in vs + tmp:
+        core.N_VDestroy(v)
