@@ -103,6 +103,11 @@ __device__ __forceinline__ double lsum(double a, double x, double b, double y)
   return (a * x) + (b * y);
 }
 
+// lsum with b = 1, whose three forms give the same bits: 1*y is y, and for
+// a = 1 the sum x + y, for a = -1 the difference y - x is what each rounds
+// (they differ only in the sign of an exact zero for a = -1)
+__device__ __forceinline__ double lsum1(double a, double x, double y) { return (a * x) + y; }
+
 __device__ __forceinline__ double sqrt0(double v) { return (v <= 0.0) ? 0.0 : sqrt(v); }
 
 // wavefront-level ordering point for a group's LDS exchange
@@ -137,8 +142,8 @@ struct Sys
   double ewt, acor, tempv, ftemp, y, delta, ysav;
   // Newton-matrix factor row held by this lane, and its physical row
   T lu[M];
-  int pos;
-  float rinv; // FP32 factors: 1 / this lane's diagonal entry
+  float rinv; // FP32 factors, groups of 32 and 64 lanes: 1 / this lane's diagonal entry
+  double dg, dr; // otherwise: this lane's diagonal entry and its reciprocal
   // integrator scalars (uniform across the group)
   double tn, h, hscale, hprime, eta, hu, h0u;
   double rl1, gamma, gammap, gamrat, crate, delp, acnrm;
@@ -329,35 +334,47 @@ __device__ __forceinline__ double g_rhs(const Grp<M, T>& g, double yi)
   gsync();
   if (g.valid) { g.red[g.i] = yi; }
   gsync();
+  // this lane's first four terms, read beside the reactions' operands
+  const int e0 = g.valid ? g.soff[g.i] : 0;
+  const int e1 = g.valid ? g.soff[g.i + 1] : 0;
+  int code[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) { code[q] = (e0 + q < e1) ? g.sent[e0 + q] : 0; }
+  // two reactions per lane in flight (R = 1.5 m makes two passes of one)
   const int R = g.a->R;
-  for (int r = g.i; r < R; r += G)
+  for (int r = g.i; r < R; r += 2 * G)
   {
-    const int4 q   = *reinterpret_cast<const int4*>(g.idx + 4 * r);
-    const double wf = (g.kf[r] * g.red[q.x]) * g.red[q.y];
-    const double wb = (g.kb[r] * g.red[q.z]) * g.red[q.w];
-    g.wbuf[r]       = wf - wb;
+    const bool two   = r + G < R;
+    const int r1     = two ? r + G : r;
+    const int4 q     = *reinterpret_cast<const int4*>(g.idx + 4 * r);
+    const int4 p     = *reinterpret_cast<const int4*>(g.idx + 4 * r1);
+    const double kf0 = g.kf[r], kb0 = g.kb[r], kf1 = g.kf[r1], kb1 = g.kb[r1];
+    const double wf0 = (kf0 * g.red[q.x]) * g.red[q.y];
+    const double wb0 = (kb0 * g.red[q.z]) * g.red[q.w];
+    const double wf1 = (kf1 * g.red[p.x]) * g.red[p.y];
+    const double wb1 = (kb1 * g.red[p.z]) * g.red[p.w];
+    g.wbuf[r]        = wf0 - wb0;
+    if (two) { g.wbuf[r1] = wf1 - wb1; }
   }
   gsync();
   double f = 0.0;
-  if (g.valid)
+  // four terms per pass: their rates and the next pass's codes are read
+  // together (independent LDS reads in flight), then added in term order
+  for (int e = e0; e < e1; e += 4)
   {
-    // four terms per pass: their codes, then their rates, are read together
-    // (independent LDS reads in flight), then added in term order
-    const int e1 = g.soff[g.i + 1];
-    for (int e = g.soff[g.i]; e < e1; e += 4)
+    double w[4];
+    int next[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) { w[q] = g.wbuf[code[q] >> 2]; }
+#pragma unroll
+    for (int q = 0; q < 4; q++) { next[q] = (e + 4 + q < e1) ? g.sent[e + 4 + q] : 0; }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
     {
-      int code[4];
-      double w[4];
-#pragma unroll
-      for (int q = 0; q < 4; q++) { code[q] = (e + q < e1) ? g.sent[e + q] : 0; }
-#pragma unroll
-      for (int q = 0; q < 4; q++) { w[q] = g.wbuf[code[q] >> 2]; }
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-      {
-        if (e + q < e1) { f = ((code[q] & 3) < 2) ? f - w[q] : f + w[q]; }
-      }
+      if (e + q < e1) { f = ((code[q] & 3) < 2) ? f - w[q] : f + w[q]; }
     }
+#pragma unroll
+    for (int q = 0; q < 4; q++) { code[q] = next[q]; }
   }
   gsync();
   BDF_PH_FENCE(f);
@@ -383,20 +400,41 @@ __device__ __forceinline__ void g_newton_matrix(const Grp<M, T>& g, double yj, d
   {
 #pragma unroll
     for (int j = 0; j < M; j++) { row[j] = (T)0; }
-    const int e1 = g.soff[g.i + 1];
-    for (int e = g.soff[g.i]; e < e1; e++)
+    // each term's operands are read while the one before it updates the row
+    const int e0 = g.soff[g.i], e1 = g.soff[g.i + 1];
+    struct Term
     {
-      const int code = g.sent[e];
-      const int r = code >> 2, t = code & 3;
-      int ix[4]    = {idx[4 * r], idx[4 * r + 1], idx[4 * r + 2], idx[4 * r + 3]};
-      double kfv   = g.kf[r], kbv = g.kb[r];
-      double dw[4] = {kfv * g.red[ix[1]], kfv * g.red[ix[0]], -(kbv * g.red[ix[3]]),
-                      -(kbv * g.red[ix[2]])};
-#pragma unroll
-      for (int q = 0; q < 4; q++)
+      int4 ix;
+      double dw[4];
+      bool loss;
+    };
+    auto term = [&](int e) {
+      Term u;
+      const int code   = g.sent[e];
+      const int r      = code >> 2;
+      u.ix             = *reinterpret_cast<const int4*>(idx + 4 * r);
+      const double kfv = g.kf[r], kbv = g.kb[r];
+      u.dw[0] = kfv * g.red[u.ix.y];
+      u.dw[1] = kfv * g.red[u.ix.x];
+      u.dw[2] = -(kbv * g.red[u.ix.w]);
+      u.dw[3] = -(kbv * g.red[u.ix.z]);
+      u.loss  = (code & 3) < 2;
+      return u;
+    };
+    if (e0 < e1)
+    {
+      Term u = term(e0);
+      for (int e = e0; e < e1; e++)
       {
-        const T v  = (T)dw[q];
-        row[ix[q]] = (t < 2) ? (row[ix[q]] - v) : (row[ix[q]] + v);
+        const Term v    = term(e + 1 < e1 ? e + 1 : e);
+        const int ix[4] = {u.ix.x, u.ix.y, u.ix.z, u.ix.w};
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+          const T d  = (T)u.dw[q];
+          row[ix[q]] = u.loss ? (row[ix[q]] - d) : (row[ix[q]] + d);
+        }
+        u = v;
       }
     }
   }
@@ -437,44 +475,63 @@ __device__ __forceinline__ float g_lane_value(float b, int k)
   }
 }
 
-// pivot search: (value, row) maximum over the group, ties to the smaller row
-using sunamd_lane::g_argmax;
-
-
-// unsigned maximum over a G-lane group (every lane ends with it)
-template <int G>
-__device__ __forceinline__ unsigned g_max_u32(unsigned v)
+// The state's arrays (Nordsieck columns, factor rows) stay in registers only
+// while every access uses a constant index.  A runtime index is resolved by
+// value: each entry is passed through an empty asm so the optimiser cannot
+// turn the choice back into an indexed load from the state struct (which would
+// move the whole integrator state to scratch memory).
+__device__ __forceinline__ double opaque(double x)
 {
-  auto mx = [](unsigned a, unsigned b) { return a > b ? a : b; };
-  if constexpr (G >= 2) { v = mx(v, (unsigned)dpp_i<0xB1>((int)v)); }
-  if constexpr (G >= 4) { v = mx(v, (unsigned)dpp_i<0x4E>((int)v)); }
-  if constexpr (G >= 8) { v = mx(v, (unsigned)dpp_i<0x141>((int)v)); }
-  if constexpr (G >= 16) { v = mx(v, (unsigned)dpp_i<0x140>((int)v)); }
-  if constexpr (G >= 32)
-  {
-    const unsigned r0 = (unsigned)__builtin_amdgcn_readlane((int)v, 0);
-    const unsigned r1 = (unsigned)__builtin_amdgcn_readlane((int)v, 16);
-    const unsigned r2 = (unsigned)__builtin_amdgcn_readlane((int)v, 32);
-    const unsigned r3 = (unsigned)__builtin_amdgcn_readlane((int)v, 48);
-    const unsigned lo = mx(r0, r1), hi = mx(r2, r3);
-    if constexpr (G == 64) { v = mx(lo, hi); }
-    else { v = (__lane_id() >= 32) ? hi : lo; }
-  }
-  return v;
+  asm("" : "+v"(x));
+  return x;
+}
+
+// lane k of each group to all of its lanes: lane reads for groups of 32 and 64
+// (few wavefronts per SIMD here, so a shuffle's LDS round trip is not hidden),
+// DPP for smaller ones
+template <int G, int K>
+__device__ __forceinline__ double g_from(double x)
+{
+  if constexpr (G >= 32) { return g_lane_value<G>(x, K); }
+  else { return sunamd_lane::g_bcast<G, K>(x); }
+}
+
+// the solves' early-known part: this lane's diagonal entry and its reciprocal
+template <int M, typename T>
+__device__ __forceinline__ void g_diagonal(const Grp<M, T>& g, Sys<M, T>& S)
+{
+  constexpr int G = pow2ceil(M);
+  T dt            = S.lu[0];
+  sunamd_lane::static_for<1, M>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    dt              = sunamd_lane::lane_is<G, j>() ? S.lu[j] : dt;
+  });
+  const double d = (double)dt;
+  S.dg = d;
+  S.dr = 1.0 / d;
 }
 
 // ---- LU of the group's matrix (rows in lanes, implicit pivoting) ---------
+// The FP64 form follows the dense GETRF operation by operation; as in the
+// block solver's k_getrf, the pivot search exchanges one word per level, the
+// pivot's reciprocal is formed beside it and (groups of up to 32 lanes) the
+// zero test is made once per column.
+// What bounds the integrator: the FP32 form's VALU issue (three wavefronts per
+// SIMD keep it 91 % busy, 3000 vector instructions per step), the FP64 form's
+// chains of dependent operations and LDS round trips (two per SIMD).  This
+// factorisation, the solves below, lsum1, the operands read ahead in g_rhs and
+// g_newton_matrix and the constant lane masks together took the uneven batch
+// of 65536 systems from 181 to 165 ms (FP64) and from 85.7 to 81.4 ms (FP32).
 template <int M, typename T>
 __device__ __forceinline__ int g_getrf(const Grp<M, T>& g, Sys<M, T>& S)
 {
   constexpr int G = pow2ceil(M);
   int pos  = g.i;
   int fail = 0;
-#pragma unroll
-  for (int k = 0; k < M; k++)
-  {
-    T v;
-    int bp;
+  // (static_for, not an unrolled loop: the larger bodies would leave the loop
+  // rolled and the rows in scratch memory)
+  sunamd_lane::static_for<0, M>([&](auto kc) {
+    constexpr int k = decltype(kc)::value;
     if constexpr (kFastFactor<T>)
     {
       // one unsigned maximum on |a_ik|'s bits with the low six replaced by
@@ -482,55 +539,13 @@ __device__ __forceinline__ int g_getrf(const Grp<M, T>& g, Sys<M, T>& S)
       const unsigned key = (g.valid && pos >= k)
                              ? ((__float_as_uint(fabsf((float)S.lu[k])) & ~63u) | (unsigned)(63 - pos))
                              : 0u;
-      const unsigned mk = g_max_u32<G>(key);
-      v  = (T)__uint_as_float(mk & ~63u);
-      bp = 63 - (int)(mk & 63u);
-    }
-    else
-    {
-      v  = (g.valid && pos >= k) ? (T)fabs((double)S.lu[k]) : (T)-1;
-      bp = g.valid ? pos : INT_MAX;
-      g_argmax<G>(v, bp);
-    }
-    if (v == (T)0 && fail == 0) { fail = k + 1; }
-    if (pos == k) { pos = bp; }
-    else if (pos == bp) { pos = k; }
-    if constexpr (G == 64)
-    {
-      // one system per wavefront: the pivot row's lane is wavefront-uniform,
-      // its entries are read straight from that lane's registers
-      const unsigned long long holder = __ballot(g.valid && pos == k);
-      const int pl  = __builtin_amdgcn_readfirstlane(__ffsll((long long)holder) - 1) & 63;
-      const bool up = g.valid && pos > k && fail == 0;
-      const T pk    = readlane_d(S.lu[k], pl);
-      if constexpr (kFastFactor<T>)
-      {
-        // single precision: multiplier 0 on the rows not updated, fused
-        // multiply-add, no zero test
-        const T l = up ? S.lu[k] * ((T)1 / pk) : (T)0;
-        if (up) { S.lu[k] = l; }
-#pragma unroll
-        for (int j = k + 1; j < M; j++) { S.lu[j] = __builtin_fmaf(-readlane_d(S.lu[j], pl), l, S.lu[j]); }
-      }
-      else
-      {
-        T l = (T)0;
-        if (up)
-        {
-          const T mult = (T)1 / pk;
-          l            = S.lu[k] * mult;
-          S.lu[k]      = l;
-        }
-#pragma unroll
-        for (int j = k + 1; j < M; j++)
-        {
-          const T pj = readlane_d(S.lu[j], pl);
-          if (up && pj != (T)0) { S.lu[j] = S.lu[j] - pj * l; }
-        }
-      }
-    }
-    else
-    {
+      const unsigned mk = sunamd_lane::g_umax<G>(key);
+      const int bp      = 63 - (int)(mk & 63u);
+      if ((mk & ~63u) == 0 && fail == 0) { fail = k + 1; }
+      if (pos == k) { pos = bp; }
+      else if (pos == bp) { pos = k; }
+      // single precision: multiplier 0 on the rows not updated, fused
+      // multiply-add, no zero test
       gsync();
       if (g.valid && pos == k)
       {
@@ -539,56 +554,121 @@ __device__ __forceinline__ int g_getrf(const Grp<M, T>& g, Sys<M, T>& S)
       }
       gsync();
       const bool up = g.valid && pos > k && fail == 0;
-      if constexpr (kFastFactor<T>)
-      {
-        const T l = up ? S.lu[k] * ((T)1 / g.prow[k]) : (T)0;
-        if (up) { S.lu[k] = l; }
+      const T l     = up ? S.lu[k] * ((T)1 / g.prow[k]) : (T)0;
+      if (up) { S.lu[k] = l; }
 #pragma unroll
-        for (int j = k + 1; j < M; j++) { S.lu[j] = __builtin_fmaf(-g.prow[j], l, S.lu[j]); }
-      }
-      else if (up)
+      for (int j = k + 1; j < M; j++) { S.lu[j] = __builtin_fmaf(-g.prow[j], l, S.lu[j]); }
+    }
+    else
+    {
+      const T rk     = (T)1 / S.lu[k];
+      const bool win = sunamd_lane::g_pivot<G>(S.lu[k], g.valid && pos >= k, pos, k, g.base);
+      if constexpr (G == 64)
       {
-        const T mult = (T)1 / g.prow[k];
-        const T l    = S.lu[k] * mult;
-        S.lu[k]      = l;
+        // one system per wavefront: the pivot row's lane is wavefront-uniform,
+        // its entries are read straight from that lane's registers (rows of
+        // 48 and 64 doubles leave none for a pivot row on its way from LDS)
+        const int pl = __builtin_amdgcn_readfirstlane(
+                         __ffsll((long long)sunamd_lane::ballot(win)) - 1) & 63;
+        const int bp = __builtin_amdgcn_readlane(pos, pl);
+        const T pk   = readlane_d(S.lu[k], pl);
+        const T mult = readlane_d(rk, pl);
+        if (pk == (T)0 && fail == 0) { fail = k + 1; }
+        if (win) { pos = k; }
+        else if (pos == k) { pos = bp; }
+        const bool up = g.valid && pos > k && fail == 0;
+        T l           = (T)0;
+        if (up)
+        {
+          l       = S.lu[k] * mult;
+          S.lu[k] = l;
+        }
 #pragma unroll
         for (int j = k + 1; j < M; j++)
         {
-          const T pj = g.prow[j];
-          if (pj != (T)0) { S.lu[j] = S.lu[j] - pj * l; }
+          const T pj = readlane_d(S.lu[j], pl);
+          if (up && pj != (T)0) { S.lu[j] = S.lu[j] - pj * l; }
+        }
+      }
+      else
+      {
+        // the pivot row publishes columns k+1..M-1, its reciprocal in column
+        // k's place, and the position it came from (64 added to it for a zero
+        // pivot)
+        gsync();
+        if (win)
+        {
+#pragma unroll
+          for (int j = k + 1; j < M; j++) { g.prow[j] = S.lu[j]; }
+          g.prow[k] = rk;
+          g.inv[0]  = pos | (S.lu[k] == (T)0 ? 64 : 0);
+        }
+        gsync();
+        const int pp = g.inv[0];
+        const T mult = g.prow[k];
+        const T mine = g.prow[g.i];
+        if (pp >= 64 && fail == 0) { fail = k + 1; }
+        if (win) { pos = k; }
+        else if (pos == k) { pos = pp & 63; }
+        const bool up    = g.valid && pos > k && fail == 0;
+        const bool zeros = sunamd_lane::ballot(g.valid && g.i > k && mine == (T)0) != 0;
+        T l              = (T)0;
+        if (up)
+        {
+          l       = S.lu[k] * mult;
+          S.lu[k] = l;
+        }
+        if (!zeros)
+        {
+          if (up)
+          {
+#pragma unroll
+            for (int j = k + 1; j < M; j++) { S.lu[j] = S.lu[j] - g.prow[j] * l; }
+          }
+        }
+        // (two ifs, not if / else: the entries then stay in their registers)
+        if (zeros)
+        {
+          if (up)
+          {
+#pragma unroll
+            for (int j = k + 1; j < M; j++)
+            {
+              const T pj = g.prow[j];
+              if (pj != (T)0) { S.lu[j] = S.lu[j] - pj * l; }
+            }
+          }
         }
       }
     }
-  }
+  });
   gsync();
   if (g.valid) { g.inv[pos] = g.i; }
   gsync();
-  S.pos = pos;
-  if constexpr (G >= 32)
+  // move physical row j to lane base+j, so the solves read row k's element
+  // from a fixed lane
+  const int src = g.base + g.inv[g.valid ? g.i : 0];
+#pragma unroll
+  for (int j = 0; j < M; j++) { S.lu[j] = __shfl(S.lu[j], src, 64); }
+  if constexpr (kFastFactor<T> && G >= 32)
   {
-    // one or two systems per wavefront: move physical row j to lane base+j,
-    // so the solves read row k's element from a fixed lane
-    const int src = g.base + g.inv[g.valid ? g.i : 0];
-#pragma unroll
-    for (int j = 0; j < M; j++) { S.lu[j] = __shfl(S.lu[j], src, 64); }
-    S.pos = g.i;
-    if constexpr (kFastFactor<T>)
-    {
-      // single precision: keep 1/u_ii per lane and store the strict upper
-      // part column-scaled, u_ij / u_jj, so the backward solve's chain is a
-      // lane read and a fused multiply-add per column
-      float d = S.lu[0];
-#pragma unroll
-      for (int j = 1; j < M; j++) { d = (j == g.i) ? S.lu[j] : d; }
-      S.rinv = 1.0f / d;
-#pragma unroll
-      for (int j = 1; j < M; j++)
-      {
-        const float rj = g_lane_value<G>(S.rinv, j);
-        S.lu[j]        = (j > g.i) ? S.lu[j] * rj : S.lu[j];
-      }
-    }
+    // single precision: keep 1/u_ii per lane and store the strict upper
+    // part column-scaled, u_ij / u_jj, so the backward solve's chain is a
+    // lane read and a fused multiply-add per column
+    using namespace sunamd_lane;
+    float d = S.lu[0];
+    static_for<1, M>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      d               = lane_is<G, j>() ? S.lu[j] : d;
+    });
+    S.rinv = 1.0f / d;
+    static_for<1, M>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      const float rj  = g_lane_value<G>(S.rinv, j);
+      S.lu[j]         = lane_below<G, j>() ? S.lu[j] * rj : S.lu[j];
+    });
   }
+  else { g_diagonal(g, S); }
   return fail;
 }
 
@@ -596,70 +676,73 @@ __device__ __forceinline__ int g_getrf(const Grp<M, T>& g, Sys<M, T>& S)
 template <int M, typename T>
 __device__ __forceinline__ double g_getrs(const Grp<M, T>& g, const Sys<M, T>& S, double b)
 {
-  // the row swaps carried logical row r to physical row pos_r, and b's
-  // element r to the same position: lane r already holds b'[pos_r]
-  const int pos = S.pos;
+  // the row swaps carried logical row r to physical row pos_r and b's element
+  // r to the same position; rows sit in lane order (physical row j in lane
+  // base+j): gather b' (b's element of row j is held by the lane the row came
+  // from), then read row k's element from lane base+k; x_i ends in lane base+i
   constexpr int G = pow2ceil(M);
-  if constexpr (G >= 32)
+  b = __shfl(b, g.base + g.inv[g.valid ? g.i : 0], 64);
+  if constexpr (kFastFactor<T> && G >= 32)
   {
-    // rows sit in lane order (physical row j in lane base+j): gather b' (b's
-    // element of row j is held by the lane the row came from), then read
-    // row k's element from lane base+k; x_i ends in lane base+i
-    b = __shfl(b, g.base + g.inv[g.valid ? g.i : 0], 64);
-    if constexpr (kFastFactor<T>)
-    {
-      // single-precision solve: multipliers selected off the dependency
-      // chain (0 on lanes a column does not update), U column-scaled
-      float x = (float)b;
-#pragma unroll
-      for (int k = 0; k < M - 1; k++)
-      {
-        const float lk = (g.i > k) ? S.lu[k] : 0.0f;
-        x              = __builtin_fmaf(-lk, g_lane_value<G>(x, k), x);
-      }
-#pragma unroll
-      for (int k = M - 1; k > 0; k--)
-      {
-        const float uk = (g.i < k) ? S.lu[k] : 0.0f;
-        x              = __builtin_fmaf(-uk, g_lane_value<G>(x, k), x);
-      }
-      return (double)(x * S.rinv);
-    }
-#pragma unroll
-    for (int k = 0; k < M - 1; k++)
-    {
-      const double bk = g_lane_value<G>(b, k);
-      if (g.i > k) { b = b - (double)S.lu[k] * bk; }
-    }
-#pragma unroll
-    for (int k = M - 1; k > 0; k--)
-    {
-      if (g.i == k) { b = b / (double)S.lu[k]; }
-      const double bk = g_lane_value<G>(b, k);
-      if (g.i < k) { b = b - (double)S.lu[k] * bk; }
-    }
-    if (g.i == 0) { b = b / (double)S.lu[0]; }
-    return b;
+    // single-precision solve: multipliers selected off the dependency
+    // chain (0 on lanes a column does not update), U column-scaled
+    using namespace sunamd_lane;
+    float x = (float)b;
+    static_for<0, M - 1>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      const float lk  = lane_above<G, k>() ? S.lu[k] : 0.0f;
+      x               = __builtin_fmaf(-lk, g_lane_value<G>(x, k), x);
+    });
+    static_for<0, M - 1>([&](auto kc) {
+      constexpr int k = M - 1 - decltype(kc)::value;
+      const float uk  = lane_below<G, k>() ? S.lu[k] : 0.0f;
+      x               = __builtin_fmaf(-uk, g_lane_value<G>(x, k), x);
+    });
+    return (double)(x * S.rinv);
   }
   else
   {
-#pragma unroll
-    for (int k = 0; k < M - 1; k++)
+    using sunamd_lane::quotient;
+    using sunamd_lane::quotient_safe;
+    using sunamd_lane::static_for;
+    static_for<0, M - 1>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      const double bk = g_from<G, k>(b);
+      if (sunamd_lane::lane_above<G, k>()) { b = b - (double)S.lu[k] * bk; }
+    });
+    // U x = y: a lane's entry is the quotient of b and its diagonal, formed
+    // where it is broadcast and once more at the end; b stays the numerator.
+    // A quotient is six operations from the diagonal's reciprocal (correctly
+    // rounded, see lane_ops.h) where a division is about eleven in a chain
+    // of M - 1 of them.
+    const double y = b;
+    static_for<0, M - 1>([&](auto kc) {
+      constexpr int k = M - 1 - decltype(kc)::value;
+      const double xk = g_from<G, k>(quotient(b, S.dg, S.dr));
+      if (sunamd_lane::lane_below<G, k>()) { b = b - (double)S.lu[k] * xk; }
+    });
+    double x = quotient(b, S.dg, S.dr);
+    if (sunamd_lane::ballot(g.valid && !(quotient_safe(S.dg) && (b == 0.0 || quotient_safe(b)))) != 0)
     {
-      double bk = __shfl(b, g.base + g.inv[k], 64);
-      if (pos > k) { b = b - (double)S.lu[k] * bk; }
-    }
+      // outside the quotient's range: the sweep with divisions
+      b = y;
+#pragma unroll 1
+      for (int k = M - 1; k > 0; k--)
+      {
+        const double xk = __shfl(b / S.dg, g.base + k, 64);
+        double lk       = opaque((double)S.lu[M > 1 ? 1 : 0]);
 #pragma unroll
-    for (int k = M - 1; k > 0; k--)
-    {
-      if (pos == k) { b = b / (double)S.lu[k]; }
-      double bk = __shfl(b, g.base + g.inv[k], 64);
-      if (pos < k) { b = b - (double)S.lu[k] * bk; }
+        for (int j = 2; j < M; j++)
+        {
+          const double lj = opaque((double)S.lu[j]);
+          lk              = (j == k) ? lj : lk;
+        }
+        if (g.i < k) { b = b - lk * xk; }
+      }
+      x = b / S.dg;
     }
+    return x;
   }
-  if (pos == 0) { b = b / (double)S.lu[0]; }
-  // variable i sits in the lane holding physical row i
-  return __shfl(b, g.base + g.inv[g.valid ? g.i : 0], 64);
 }
 
 // ---- integrator pieces -----------------------------------------------------
@@ -670,17 +753,6 @@ __device__ __forceinline__ double g_ewt(const Grp<M, T>& g, double yi)
   t        = g.a->rtol * t;
   t        = t + g.a->atol;
   return 1.0 / t;
-}
-
-// The Nordsieck columns stay in registers only while every access uses a
-// constant index.  A runtime column index is resolved by value: each column is
-// passed through an empty asm so the optimiser cannot turn the choice back
-// into an indexed load from the state struct (which would move the whole
-// integrator state to scratch memory).
-__device__ __forceinline__ double opaque(double x)
-{
-  asm("" : "+v"(x));
-  return x;
 }
 
 template <int M, typename T>
@@ -745,7 +817,7 @@ __device__ __forceinline__ void g_increase_bdf(const Grp<M, T>& g, Sys<M, T>& S)
 #pragma unroll
   for (int j = 2; j <= QMAX; j++)
   {
-    if (j <= S.q) { S.zn[j] = lsum(l[j], zL, 1.0, S.zn[j]); }
+    if (j <= S.q) { S.zn[j] = lsum1(l[j], zL, S.zn[j]); }
   }
 }
 
@@ -905,11 +977,11 @@ __device__ __forceinline__ void g_set(const Grp<M, T>& g, Sys<M, T>& S, long nst
 template <int M, typename T>
 __device__ __forceinline__ void g_residual(const Grp<M, T>& g, Sys<M, T>& S)
 {
-  S.y     = lsum(1.0, S.zn[0], 1.0, S.acor);
+  S.y     = S.zn[0] + S.acor;
   S.ftemp = g_rhs(g, S.y);
   S.nfe++;
-  double res = lsum(S.rl1, S.zn[1], 1.0, S.acor);
-  S.delta    = lsum(-S.gamma, S.ftemp, 1.0, res);
+  double res = lsum1(S.rl1, S.zn[1], S.acor);
+  S.delta    = lsum1(-S.gamma, S.ftemp, res);
 }
 
 // linear-solver setup (cvNlsLSetup + cvLsSetup + cvLsLinSys + GETRF)
@@ -1014,7 +1086,7 @@ __device__ __forceinline__ int g_newton(const Grp<M, T>& g, Sys<M, T>& S, bool c
       niters++;
       S.delta = -1.0 * S.delta;
       g_lsolve(g, S);
-      S.acor = lsum(1.0, S.acor, 1.0, S.delta);
+      S.acor = S.acor + S.delta;
       retval = g_ctest(g, S, curiter, tol, nonzero_start);
       curiter++;
       if (retval == CV_SUCCESS)
@@ -1280,7 +1352,7 @@ __device__ __forceinline__ int g_nls(const Grp<M, T>& g, Sys<M, T>& S, int nflag
   {
     g_log_pair(g, S);
   }
-  S.y = lsum(1.0, S.zn[0], 1.0, S.acor);
+  S.y = S.zn[0] + S.acor;
   if (!S.acnrmcur) { S.acnrm = g_wrms(g, S.acor, S.ewt); }
   return flag;
 }
@@ -1380,7 +1452,7 @@ __device__ __forceinline__ void g_complete_step(const Grp<M, T>& g, Sys<M, T>& S
 #pragma unroll
   for (int j = 0; j <= QMAX; j++)
   {
-    if (j <= S.q) { S.zn[j] = lsum(l[j], S.acor, 1.0, S.zn[j]); }
+    if (j <= S.q) { S.zn[j] = lsum1(l[j], S.acor, S.zn[j]); }
   }
   S.qwait--;
   if ((S.qwait == 1) && (S.q != QMAX))
@@ -1497,7 +1569,7 @@ __device__ __forceinline__ int g_hin(const Grp<M, T>& g, Sys<M, T>& S, double to
   double temp2  = fabs(S.zn[0]);
   double temp1  = g_ewt(g, S.zn[0]);
   temp1         = 1.0 / temp1;
-  temp1         = lsum(HUB_FACTOR, temp2, 1.0, temp1);
+  temp1         = lsum1(HUB_FACTOR, temp2, temp1);
   temp2         = fabs(S.zn[1]);
   temp1         = temp2 / temp1;
   double hubinv = g_maxabs(g, temp1);
@@ -1514,7 +1586,7 @@ __device__ __forceinline__ int g_hin(const Grp<M, T>& g, Sys<M, T>& S, double to
   {
     // cvYddNorm (the RHS never fails here)
     double hgs = hg * sign;
-    S.y        = lsum(hgs, S.zn[1], 1.0, S.zn[0]);
+    S.y        = lsum1(hgs, S.zn[1], S.zn[0]);
     S.tempv    = g_rhs(g, S.y);
     S.nfe++;
     S.tempv = lsum(1.0 / hgs, S.tempv, -1.0 / hgs, S.zn[1]);
@@ -1617,7 +1689,6 @@ __device__ __forceinline__ bool g_acquire(Grp<M, T>& g, Sys<M, T>& S, double tou
     S.etaq = S.etaqm1 = S.etaqp1 = S.eta = S.hprime = 0.0;
     S.qprime   = 1;
     S.convfail = CV_NO_FAILURES;
-    S.pos      = g.i;
     S.ltried = S.lused = 0;
     {
       // learned-predictor input: log10(1 + sum of k_f + k_b over the
@@ -1767,7 +1838,7 @@ __device__ __forceinline__ bool g_advance_tail(const Grp<M, T>& g, Sys<M, T>& S,
       double cj = 1.0;
       for (int i = 0; i < j; i++) { cj *= s; }
       double zj = zget(S, j);
-      z         = (j == S.q) ? cj * zj : lsum(cj, zj, 1.0, z);
+      z         = (j == S.q) ? cj * zj : lsum1(cj, zj, z);
     }
     yout = z;
     flag = CV_SUCCESS;
@@ -1790,7 +1861,7 @@ __global__ void __launch_bounds__(64, W) k_batched_bdf(BucketArgs A)
   constexpr int G   = pow2ceil(M);
   constexpr int GPW = 64 / G;
   __shared__ double s_red[64];
-  __shared__ T s_prow[64];
+  __shared__ __align__(16) T s_prow[64];
   __shared__ int s_inv[64];
   __shared__ GroupScalars s_sc[GPW];
   // dynamic LDS: per-group rate constants (GPW x 2R doubles), the network

@@ -369,47 +369,36 @@ __device__ __forceinline__ void stage_rates(const CplArgs& A, const Grp<M, T>& g
 }
 
 // the saved factorisation of a cell, as the register LU left it
-// The row permutation is kept as each lane's physical row (groups under 32
-// lanes, rows stay where the pivoting left them) or as the inverse
-// permutation the solve gathers with (32 and 64 lanes, rows moved to lane
-// order after the factorisation); the solve reads it from the group's LDS.
+// The rows are in lane order (physical row j in lane j); the row permutation
+// is kept as the inverse permutation the solve gathers with, which it reads
+// from the group's LDS.
 template <int M, typename T>
 __device__ __forceinline__ void lu_store(const CplArgs& A, const Grp<M, T>& g,
                                          const Sys<M, T>& S, const Cell<M, T>& c)
 {
-  constexpr int G = pow2ceil(M);
-  int p           = S.pos;
-  if constexpr (G >= 32) { p = g.inv[g.valid ? g.i : 0]; }
+  const int p = g.inv[g.valid ? g.i : 0];
   if (!c.lv) { return; }
   auto lu = gptr((T*)A.lu) + c.cc * (long)M * M + g.i;
 #pragma unroll
   for (int j = 0; j < M; j++) { lu[(long)j * M] = S.lu[j]; }
   gptr(A.pos)[c.e] = p;
-  if constexpr (sizeof(T) == 4) { gptr(A.rinv)[c.e] = S.rinv; }
+  if constexpr (sizeof(T) == 4 && pow2ceil(M) >= 32) { gptr(A.rinv)[c.e] = S.rinv; }
 }
 
 template <int M, typename T>
 __device__ __forceinline__ void lu_load(const CplArgs& A, const Grp<M, T>& g, Sys<M, T>& S,
                                         const Cell<M, T>& c)
 {
-  constexpr int G = pow2ceil(M);
-  const auto lu   = gptr((const T*)A.lu) + c.cc * (long)M * M + (g.valid ? g.i : 0);
+  constexpr bool scaled = sizeof(T) == 4 && pow2ceil(M) >= 32;
+  const auto lu         = gptr((const T*)A.lu) + c.cc * (long)M * M + (g.valid ? g.i : 0);
 #pragma unroll
   for (int j = 0; j < M; j++) { S.lu[j] = g.valid ? lu[(long)j * M] : (T)0; }
   const int p = g.valid ? gptr(A.pos)[c.e] : g.i;
-  if constexpr (sizeof(T) == 4) { S.rinv = g.valid ? gptr(A.rinv)[c.e] : 1.0f; }
+  if constexpr (scaled) { S.rinv = g.valid ? gptr(A.rinv)[c.e] : 1.0f; }
   gsync();
-  if constexpr (G >= 32)
-  {
-    S.pos = g.i;
-    if (g.valid) { g.inv[g.i] = p; }
-  }
-  else
-  {
-    S.pos = p;
-    if (g.valid) { g.inv[p] = g.i; }
-  }
+  if (g.valid) { g.inv[g.i] = p; }
   gsync();
+  if constexpr (!scaled) { g_diagonal(g, S); }
 }
 
 __device__ __forceinline__ void add_term(const CplArgs& A, double (&acc)[3], int k, long e,
@@ -649,7 +638,7 @@ __device__ __forceinline__ void pass_newton(const CplArgs& A, const Grp<M, T>& g
       }
     }
     if (d.acor_zero) { acor = 0.0; }
-    const double y = lsum(1.0, z[0], 1.0, acor);
+    const double y = z[0] + acor;
     if (d.setup)
     {
       double ys;
@@ -666,12 +655,12 @@ __device__ __forceinline__ void pass_newton(const CplArgs& A, const Grp<M, T>& g
       lu_store(A, g, S, c);
     }
     const double f = regs ? rhs_regs(A, g, y, kr, br) : g_rhs(g, y);
-    const double res = lsum(d.rl1, z[1], 1.0, acor);
-    double delta     = lsum(-d.gamma, f, 1.0, res);
+    const double res = lsum1(d.rl1, z[1], acor);
+    double delta     = lsum1(-d.gamma, f, res);
     delta            = -1.0 * delta;
     delta            = g_getrs(g, S, delta);
     if (d.gscale != 1.0) { delta = d.gscale * delta; }
-    acor = lsum(1.0, acor, 1.0, delta);
+    acor = acor + delta;
     if (c.lv) { gptr(A.acor)[c.e] = acor; }
     add_term(A, acc, 0, c.e, c.lv, delta, w, gen);
     add_term(A, acc, 1, c.e, c.lv, acor, w, gen);
@@ -760,7 +749,7 @@ __global__ void __launch_bounds__(64 * cpl_waves<M>(), 2) k_coupled_bdf(const Cp
   constexpr int CW  = cpl_waves<M>();
   constexpr int CT  = 64 * CW;
   __shared__ double s_red[CW][64];
-  __shared__ T s_prow[CW][64];
+  __shared__ __align__(16) T s_prow[CW][64];
   __shared__ int s_inv[CW][64];
   __shared__ GroupScalars s_sc[CW * GPW];
   __shared__ double s_w[CW][NRED];
@@ -814,8 +803,8 @@ __global__ void __launch_bounds__(64 * cpl_waves<M>(), 2) k_coupled_bdf(const Cp
   else { g.jrow = (T*)(area + 2 * A.R) + (long)(g.valid ? g.i : 0) * (M + 1); }
   g.cell  = 0;
   Sys<M, T> S;
-  S.pos  = g.i;
   S.rinv = 1.0f;
+  S.dg = S.dr = 1.0;
 
   // this wavefront's cells: chunks [ch0, ch1) of GPW consecutive cells
   const long NWV = (long)A.nwg * CW;
@@ -915,7 +904,7 @@ __global__ void __launch_bounds__(64 * cpl_waves<M>(), 2) k_coupled_bdf(const Cp
             stage_rates(A, g, c.cc);
             const double z0 = c.lv ? gptr(A.zn)[c.e] : 0.0;
             const double z1 = c.lv ? gptr(A.zn)[N + c.e] : 0.0;
-            const double y  = lsum(hgs, z1, 1.0, z0);
+            const double y  = lsum1(hgs, z1, z0);
             const double f  = g_rhs(g, y);
             const double t  = lsum(ra, f, rb, z1);
             add_term(A, a2, 0, c.e, c.lv, t, c.lv ? gptr(A.ewt)[c.e] : 0.0, gen);

@@ -196,6 +196,46 @@ __device__ __forceinline__ bool g_pivot(T ak, bool cand, int pos, int k, int bas
   return win;
 }
 
+// ---- constant sets of lanes ---------------------------------------------------
+// Lanes whose index in their G-lane group is above / below / equal to k, as a
+// condition: a constant mask moved into scalar registers where it is used (the
+// moves are volatile: as plain constants the masks of a whole sweep are
+// hoisted out of the integrators' step loop and spilled to vector lanes),
+// instead of a vector compare.
+template <int G>
+constexpr unsigned long long lanes_mask(int lo, int hi)
+{
+  unsigned long long m = 0;
+  for (int l = 0; l < 64; l++)
+  {
+    if (l % G >= lo && l % G < hi) { m |= 1ULL << l; }
+  }
+  return m;
+}
+template <unsigned long long MASK>
+__device__ __forceinline__ bool in_lanes()
+{
+  unsigned lo, hi;
+  asm volatile("s_mov_b32 %0, %1" : "=s"(lo) : "i"((int)(MASK & 0xffffffffULL)));
+  asm volatile("s_mov_b32 %0, %1" : "=s"(hi) : "i"((int)(MASK >> 32)));
+  return __builtin_amdgcn_inverse_ballot_w64(((unsigned long long)hi << 32) | lo);
+}
+template <int G, int K>
+__device__ __forceinline__ bool lane_above()
+{
+  return in_lanes<lanes_mask<G>(K + 1, G)>();
+}
+template <int G, int K>
+__device__ __forceinline__ bool lane_below()
+{
+  return in_lanes<lanes_mask<G>(0, K)>();
+}
+template <int G, int K>
+__device__ __forceinline__ bool lane_is()
+{
+  return in_lanes<lanes_mask<G>(K, K + 1)>();
+}
+
 // ---- lane k of each G-lane group to all of its lanes, k a constant ----------
 // A lane read for groups of 64; an LDS shuffle for 32 (one instruction beside
 // the VALU, where two lane reads and a select are three in it); DPP for

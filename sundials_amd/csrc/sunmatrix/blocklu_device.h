@@ -366,21 +366,23 @@ __global__ void __launch_bounds__(64 * LU_WAVES) k_getrs(const T* __restrict__ F
     constexpr int k = decltype(kc)::value;
     if (RT && k >= m - 1) { return; }
     const double bk = g_bcast<G, k>(bi);
-    if (r > k) { bi = bi - (double)lu[k] * bk; }
+    if (lane_above<G, k>()) { bi = bi - (double)lu[k] * bk; }
   });
   // U x = y.  A lane's own entry is its quotient bi / d, formed where it is
   // broadcast and once more at the end; bi stays the numerator.
   const double y = bi;
   T dt           = lu[0];
-#pragma unroll
-  for (int j = 1; j < M; j++) { dt = (j == r) ? lu[j] : dt; }
+  static_for<1, M>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    dt              = lane_is<G, j>() ? lu[j] : dt;
+  });
   const double d    = (double)dt;
   const double rinv = 1.0 / d;
   static_for<0, M - 1>([&](auto kc) {
     constexpr int k = M - 1 - decltype(kc)::value;
     if (RT && k >= m) { return; }
     const double xk = g_bcast<G, k>(quotient(bi, d, rinv));
-    if (r < k) { bi = bi - (double)lu[k] * xk; }
+    if (lane_below<G, k>()) { bi = bi - (double)lu[k] * xk; }
   });
   double xi = quotient(bi, d, rinv);
   if (ballot(valid && !(quotient_safe(d) && (bi == 0.0 || quotient_safe(bi)))) != 0)
