@@ -18,11 +18,13 @@
 #include <hip/hip_runtime.h>
 
 #include <chrono>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 
 #include "../batched/coupled_device.h"
+#include "../core/lane_ops.h"
 #include "../core/profiler_internal.h"
 #include "sunamd/cvode_sunamd.h"
 #include "sunamd/sunamd_profiler.h"
@@ -68,7 +70,45 @@ __device__ __forceinline__ void ma_stage_tables(const int* __restrict__ idx,
   for (int t = threadIdx.x; t <= m; t += blockDim.x) { s_soff[t] = soff[t]; }
 }
 
-// f = RHS(y): per group, y (m) and the net rates w (R) in LDS
+// A cell's operands on their way from HBM while the cell before it is worked
+// on: its species of this lane and the rates of this lane's first two
+// reactions (R = 1.5 m needs no more; further ones are loaded where they are
+// used).  Lanes without a cell or a reaction read inside the arrays and drop
+// the value, so the loads are unconditional.
+struct MaNext
+{
+  double y, kf[2], kb[2];
+};
+
+__device__ __forceinline__ MaNext ma_fetch(const double* __restrict__ y,
+                                           const double* __restrict__ kf,
+                                           const double* __restrict__ kb, long cell, long ncells,
+                                           int i, int m, int G, int R)
+{
+  MaNext n;
+  const long c = cell < ncells ? cell : ncells - 1;
+  n.y          = y[c * m + (i < m ? i : m - 1)];
+#pragma unroll
+  for (int q = 0; q < 2; q++)
+  {
+    const int r = (i + q * G < R) ? i + q * G : R - 1;
+    n.kf[q]     = kf[c * R + r];
+    n.kb[q]     = kb[c * R + r];
+  }
+  return n;
+}
+
+// f = RHS(y): per group, y (m), the net rates w (R) and a zero in LDS.  One
+// wavefront per workgroup: its LDS exchanges need a wavefront-level ordering
+// point only (a workgroup barrier would also wait for the next cell's loads).
+//
+// What bounds it: LDS and VALU issue about as much as HBM (m = 32, R = 48:
+// 1280 bytes per cell; 2^18 cells in 57 us at the copy rate).  A lane's terms
+// are the same for every cell, so the first MA_TERMS of them (their rate's
+// place and sign) stay in registers instead of being read from LDS per cell:
+// 101 -> 98 us.
+constexpr int MA_TERMS = 12;
+
 __global__ void __launch_bounds__(64) k_ma_rhs(const double* __restrict__ y,
                                                double* __restrict__ f,
                                                const int* __restrict__ idx,
@@ -78,9 +118,10 @@ __global__ void __launch_bounds__(64) k_ma_rhs(const double* __restrict__ y,
                                                const double* __restrict__ kb, int m, int G,
                                                int R, long ncells)
 {
+  using sunamd_lane::wave_sync;
   extern __shared__ __align__(16) double sm[];
   const int gpw   = 64 / G;
-  const long per  = (long)((m + R + 1) & ~1);
+  const long per  = (long)((m + R + 2) & ~1);
   const int grp   = threadIdx.x / G;
   const int i     = threadIdx.x % G;
   double* ys      = sm + grp * per;
@@ -88,35 +129,77 @@ __global__ void __launch_bounds__(64) k_ma_rhs(const double* __restrict__ y,
   int* s_idx      = (int*)(sm + gpw * per);
   int* s_sent     = s_idx + 4 * R;
   int* s_soff     = s_sent + 4 * R;
+  const long step = (long)gridDim.x * gpw;
+  MaNext nx       = ma_fetch(y, kf, kb, (long)blockIdx.x * gpw + grp, ncells, i, m, G, R);
   ma_stage_tables(idx, soff, sent, s_idx, s_soff, s_sent, m, R);
   __syncthreads();
   const int e0    = (i < m) ? s_soff[i] : 0;
   const int e1    = (i < m) ? s_soff[i + 1] : 0;
   const int4* ix4 = (const int4*)s_idx;
-  // the loop bound is the workgroup's, so every lane meets every barrier
-  for (long c0 = (long)blockIdx.x * gpw; c0 < ncells; c0 += (long)gridDim.x * gpw)
+  // place of the term's rate, sign in the top bit; absent terms add ws[R] = 0
+  // (the sum starts from +0, which no sum of it with zeros leaves)
+  unsigned term[MA_TERMS];
+#pragma unroll
+  for (int q = 0; q < MA_TERMS; q++)
+  {
+    const int code = (e0 + q < e1) ? s_sent[e0 + q] : 4 * R + 2;
+    term[q]        = (unsigned)(code >> 2) | ((code & 3) < 2 ? 0x80000000u : 0u);
+  }
+  const int most = e1 - e0 < MA_TERMS ? e1 - e0 : MA_TERMS; // terms of this lane in registers
+  if (i == 0) { ws[R] = 0.0; }
+  for (long c0 = (long)blockIdx.x * gpw; c0 < ncells; c0 += step)
   {
     const long cell = c0 + grp;
     const bool live = cell < ncells;
-    if (live && i < m) { ys[i] = y[cell * m + i]; }
-    __syncthreads();
+    const MaNext nc = nx;
+    if (live && i < m) { ys[i] = nc.y; }
+    wave_sync();
+    nx = ma_fetch(y, kf, kb, cell + step, ncells, i, m, G, R);
     if (live)
     {
-      const double* kfc = kf + cell * R;
-      const double* kbc = kb + cell * R;
-      for (int r = i; r < R; r += G)
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+      {
+        const int r = i + q * G;
+        if (r < R)
+        {
+          const int4 ix   = ix4[r];
+          const double wf = (nc.kf[q] * ys[ix.x]) * ys[ix.y];
+          const double wb = (nc.kb[q] * ys[ix.z]) * ys[ix.w];
+          ws[r]           = wf - wb;
+        }
+      }
+      for (int r = i + 2 * G; r < R; r += G)
       {
         const int4 ix   = ix4[r];
-        const double wf = (kfc[r] * ys[ix.x]) * ys[ix.y];
-        const double wb = (kbc[r] * ys[ix.z]) * ys[ix.w];
+        const double wf = (kf[cell * R + r] * ys[ix.x]) * ys[ix.y];
+        const double wb = (kb[cell * R + r] * ys[ix.z]) * ys[ix.w];
         ws[r]           = wf - wb;
       }
     }
-    __syncthreads();
+    wave_sync();
     if (live && i < m)
     {
       double acc = 0.0;
-      for (int e = e0; e < e1; e++)
+#pragma unroll
+      for (int q0 = 0; q0 < MA_TERMS; q0 += 4)
+      {
+        if (q0 < most)
+        {
+          double w[4];
+#pragma unroll
+          for (int q = 0; q < 4; q++) { w[q] = ws[term[q0 + q] & 0x7fffffffu]; }
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+          {
+            // acc - w is acc + (-w)
+            const long long v = __double_as_longlong(w[q]) ^
+                                ((long long)(term[q0 + q] & 0x80000000u) << 32);
+            acc               = acc + __longlong_as_double(v);
+          }
+        }
+      }
+      for (int e = e0 + MA_TERMS; e < e1; e++)
       {
         const int code = s_sent[e];
         const double w = ws[code >> 2];
@@ -124,12 +207,28 @@ __global__ void __launch_bounds__(64) k_ma_rhs(const double* __restrict__ y,
       }
       f[cell * m + i] = acc;
     }
-    __syncthreads();
+    wave_sync();
   }
 }
 
+// one term of a Jacobian row: the reaction's species and the partial
+// derivatives of its rate, and whether the row loses by it
+struct MaTerm
+{
+  int4 ix;
+  double dw[4];
+  bool loss;
+};
+
 // J = df/dy, block column-major: per group, the block (m*m), y (m) and the
-// cell's rates (2R) in LDS
+// cell's rates (2R) in LDS.
+//
+// What bounds it: 8 m^2 bytes per cell to HBM (m = 32: 9.2 KB, 2^18 cells in
+// 0.41 ms at the copy rate) against the chain of LDS updates of a row.  So the
+// next cell's operands are fetched meanwhile, a term's operands are read while
+// the one before it updates the row, and the block is cleared as it is
+// written out (in pairs of doubles where m*m is even): 0.58 -> 0.43 ms.
+template <bool PAIRS>
 __global__ void __launch_bounds__(64) k_ma_jac(const double* __restrict__ y,
                                                double* __restrict__ J,
                                                const int* __restrict__ idx,
@@ -139,6 +238,7 @@ __global__ void __launch_bounds__(64) k_ma_jac(const double* __restrict__ y,
                                                const double* __restrict__ kb, int m, int G,
                                                int R, long ncells)
 {
+  using sunamd_lane::wave_sync;
   extern __shared__ __align__(16) double sj[];
   const int gpw   = 64 / G;
   const int mm    = m * m;
@@ -151,55 +251,93 @@ __global__ void __launch_bounds__(64) k_ma_jac(const double* __restrict__ y,
   int* s_idx      = (int*)(sj + gpw * per);
   int* s_sent     = s_idx + 4 * R;
   int* s_soff     = s_sent + 4 * R;
+  const long step = (long)gridDim.x * gpw;
+  MaNext nx       = ma_fetch(y, kf, kb, (long)blockIdx.x * gpw + grp, ncells, i, m, G, R);
   ma_stage_tables(idx, soff, sent, s_idx, s_soff, s_sent, m, R);
+  for (int e = i; e < mm; e += G) { Jl[e] = 0.0; }
   __syncthreads();
   const int e0    = (i < m) ? s_soff[i] : 0;
   const int e1    = (i < m) ? s_soff[i + 1] : 0;
   const int4* ix4 = (const int4*)s_idx;
-  for (long c0 = (long)blockIdx.x * gpw; c0 < ncells; c0 += (long)gridDim.x * gpw)
+  auto term       = [&](int e) {
+    MaTerm u;
+    const int code   = s_sent[e];
+    const int r      = code >> 2;
+    u.loss           = (code & 3) < 2;
+    u.ix             = ix4[r];
+    const double kfv = rk[r], kbv = rk[R + r];
+    u.dw[0] = kfv * ys[u.ix.y];
+    u.dw[1] = kfv * ys[u.ix.x];
+    u.dw[2] = -(kbv * ys[u.ix.w]);
+    u.dw[3] = -(kbv * ys[u.ix.z]);
+    return u;
+  };
+  for (long c0 = (long)blockIdx.x * gpw; c0 < ncells; c0 += step)
   {
     const long cell = c0 + grp;
     const bool live = cell < ncells;
     if (live)
     {
-      for (int e = i; e < mm; e += G) { Jl[e] = 0.0; }
-      if (i < m) { ys[i] = y[cell * m + i]; }
-      for (int r = i; r < R; r += G)
+      if (i < m) { ys[i] = nx.y; }
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+      {
+        const int r = i + q * G;
+        if (r < R)
+        {
+          rk[r]     = nx.kf[q];
+          rk[R + r] = nx.kb[q];
+        }
+      }
+      for (int r = i + 2 * G; r < R; r += G)
       {
         rk[r]     = kf[cell * R + r];
         rk[R + r] = kb[cell * R + r];
       }
     }
-    __syncthreads();
-    if (live && i < m)
+    wave_sync();
+    nx = ma_fetch(y, kf, kb, cell + step, ncells, i, m, G, R);
+    if (live && e0 < e1)
     {
       // row i: the terms in which species i is a target, each adding the
       // reaction's partial derivatives to the columns of its four species
+      MaTerm u = term(e0);
       for (int e = e0; e < e1; e++)
       {
-        const int code  = s_sent[e];
-        const int r     = code >> 2;
-        const bool loss = (code & 3) < 2;
-        const int4 ix   = ix4[r];
-        const double kfv = rk[r], kbv = rk[R + r];
-        const int col[4]   = {ix.x, ix.y, ix.z, ix.w};
-        const double dw[4] = {kfv * ys[ix.y], kfv * ys[ix.x], -(kbv * ys[ix.w]),
-                              -(kbv * ys[ix.z])};
+        const MaTerm v   = term(e + 1 < e1 ? e + 1 : e);
+        const int col[4] = {u.ix.x, u.ix.y, u.ix.z, u.ix.w};
 #pragma unroll
         for (int q = 0; q < 4; q++)
         {
           const int a = col[q] * m + i;
-          Jl[a]       = loss ? (Jl[a] - dw[q]) : (Jl[a] + dw[q]);
+          Jl[a]       = u.loss ? (Jl[a] - u.dw[q]) : (Jl[a] + u.dw[q]);
         }
+        u = v;
       }
     }
-    __syncthreads();
+    wave_sync();
     if (live)
     {
       double* Jc = J + cell * (long)mm;
-      for (int e = i; e < mm; e += G) { Jc[e] = Jl[e]; }
+      if (PAIRS)
+      {
+        for (int e = i; e < mm / 2; e += G)
+        {
+          double2* d = reinterpret_cast<double2*>(Jl) + e;
+          reinterpret_cast<double2*>(Jc)[e] = *d;
+          *d                                = make_double2(0.0, 0.0);
+        }
+      }
+      else
+      {
+        for (int e = i; e < mm; e += G)
+        {
+          Jc[e] = Jl[e];
+          Jl[e] = 0.0;
+        }
+      }
     }
-    __syncthreads();
+    wave_sync();
   }
 }
 
@@ -214,7 +352,7 @@ static int pow2ceil_h(int m)
 static size_t ma_rhs_lds(int m, int R)
 {
   const int gpw = 64 / pow2ceil_h(m);
-  return sizeof(double) * (size_t)gpw * (size_t)((m + R + 1) & ~1) +
+  return sizeof(double) * (size_t)gpw * (size_t)((m + R + 2) & ~1) +
          sizeof(int) * ma_table_ints(m, R);
 }
 
@@ -297,10 +435,13 @@ extern "C" void SUNAMD_MassActionDevFree(SUNAMD_MassActionDev* d)
   free(d);
 }
 
-// workgroups for a grid-stride launch: enough to fill every CU at the
-// kernel's occupancy, no more than the cells need
+// workgroups for a grid-stride launch: enough to fill every CU `rounds` times
+// at the kernel's occupancy, no more than the cells need.  The Jacobian's take
+// one round (m = 32, 2^18 cells: 431 us, 466 with two, 478 with eight -- fewer
+// table stagings, and a long run of prefetched cells each), the right-hand
+// side's four (98 us, 103 with one: its short passes leave wavefronts uneven).
 template <typename K>
-static unsigned ma_grid(K kern, size_t shm, long ncells, int gpw)
+static unsigned ma_grid(K kern, size_t shm, long ncells, int gpw, int rounds)
 {
   static int cus = 0;
   if (cus == 0)
@@ -320,7 +461,7 @@ static unsigned ma_grid(K kern, size_t shm, long ncells, int gpw)
     per_cu = 1;
   }
   const long need = (ncells + gpw - 1) / gpw;
-  const long full = 4L * per_cu * cus;
+  const long full = (long)rounds * per_cu * cus;
   return (unsigned)(need < full ? need : full);
 }
 
@@ -331,7 +472,7 @@ extern "C" int SUNAMD_MassActionRhsDevArrays(SUNAMD_MassActionDev* d, const doub
   const int gpw = 64 / G;
   const size_t shm = ma_rhs_lds(d->m, d->R);
   if (d->ncells < 1) { return 0; }
-  if (d->rhs_grid == 0) { d->rhs_grid = ma_grid(k_ma_rhs, shm, d->ncells, gpw); }
+  if (d->rhs_grid == 0) { d->rhs_grid = ma_grid(k_ma_rhs, shm, d->ncells, gpw, 4); }
   const unsigned g = d->rhs_grid;
   sunamd_prof_begin(SUNAMD_K_RHS, d->stream);
   k_ma_rhs<<<g, 64, shm, d->stream>>>(dy, df, d->idx, d->soff, d->sent, d->kf, d->kb, d->m, G,
@@ -348,10 +489,13 @@ extern "C" int SUNAMD_MassActionJacDevArrays(SUNAMD_MassActionDev* d, const doub
   const int gpw = 64 / G;
   const size_t shm = ma_jac_lds(d->m, d->R);
   if (d->ncells < 1) { return 0; }
-  if (d->jac_grid == 0) { d->jac_grid = ma_grid(k_ma_jac, shm, d->ncells, gpw); }
+  // blocks of an even number of entries start on 16 bytes if the array does
+  const bool pairs = (d->m * d->m) % 2 == 0 && ((uintptr_t)dJ & 15u) == 0;
+  auto kern        = pairs ? k_ma_jac<true> : k_ma_jac<false>;
+  if (d->jac_grid == 0) { d->jac_grid = ma_grid(k_ma_jac<true>, shm, d->ncells, gpw, 1); }
   const unsigned g = d->jac_grid;
-  k_ma_jac<<<g, 64, shm, d->stream>>>(dy, dJ, d->idx, d->soff, d->sent, d->kf, d->kb, d->m, G,
-                                      d->R, d->ncells);
+  kern<<<g, 64, shm, d->stream>>>(dy, dJ, d->idx, d->soff, d->sent, d->kf, d->kb, d->m, G, d->R,
+                                  d->ncells);
   hipError_t e = hipGetLastError();
   return (e == hipSuccess) ? 0 : hipfail(e, "jac launch");
 }
