@@ -65,16 +65,41 @@ __global__ void k_fill(double* __restrict__ a, long n, double v)
   }
 }
 
-// A = c*A + I (per element: a *= c; a += 1 on the diagonal)
-__global__ void k_scaleaddi(double* __restrict__ a, long n, long m, double c)
+// A = c*A + I (per element: a *= c; a += 1 on the diagonal), HBM-bound.  A
+// thread takes pairs of elements and carries its place in the block along (the
+// stride's remainder added, one conditional subtraction) instead of a 64-bit
+// division per element: m = 21, 50000 blocks (353 MB) 60 -> 53 us.  U: unsigned
+// while m*m fits in it.
+template <typename U>
+__global__ void __launch_bounds__(EW_BLOCK) k_scaleaddi(double* __restrict__ a, long n, long m,
+                                                        double c)
 {
-  const long mm = m * m;
-  for (long i = (long)blockIdx.x * EW_BLOCK + threadIdx.x; i < n; i += (long)gridDim.x * EW_BLOCK)
+  const U mm        = (U)m * (U)m, m1 = (U)m + 1;
+  const long first  = 2 * ((long)blockIdx.x * EW_BLOCK + threadIdx.x);
+  const long stride = 2L * gridDim.x * EW_BLOCK;
+  U at              = (U)(first % (long)mm); // place in the block
+  const U by        = (U)(stride % (long)mm);
+  for (long i = first; i < n; i += stride)
   {
-    long e   = i % mm;
-    double v = a[i] * c;
-    if (e % (m + 1) == 0) { v = v + 1.0; }
-    a[i] = v;
+    const U at1 = (at + 1 == mm) ? 0 : at + 1;
+    if (i + 1 < n)
+    {
+      double2* p = reinterpret_cast<double2*>(a + i);
+      double2 v  = *p;
+      v.x        = v.x * c;
+      v.y        = v.y * c;
+      if (at % m1 == 0) { v.x = v.x + 1.0; }
+      if (at1 % m1 == 0) { v.y = v.y + 1.0; }
+      *p = v;
+    }
+    else
+    {
+      double v = a[i] * c;
+      if (at % m1 == 0) { v = v + 1.0; }
+      a[i] = v;
+    }
+    at += by;
+    if (at >= mm) { at -= mm; }
   }
 }
 
@@ -345,7 +370,8 @@ static SUNErrCode bm_copy(SUNMatrix A, SUNMatrix B)
 static SUNErrCode bm_scaleaddi(sunrealtype c, SUNMatrix A)
 {
   long n = bm_len(A);
-  k_scaleaddi<<<ew_grid(n), EW_BLOCK, 0, BM(A)->stream>>>(BM(A)->dev, n, (long)BM(A)->m, c);
+  auto kern = BM(A)->m < 65536 ? k_scaleaddi<unsigned> : k_scaleaddi<unsigned long>;
+  kern<<<ew_grid((n + 1) / 2), EW_BLOCK, 0, BM(A)->stream>>>(BM(A)->dev, n, (long)BM(A)->m, c);
   LAUNCHCHK(A->sunctx);
   return SUN_SUCCESS;
 }
