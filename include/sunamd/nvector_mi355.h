@@ -106,6 +106,15 @@ int cvEwtSetSV_fused_Mi355(sunbooleantype atolMin0, sunrealtype reltol, N_Vector
 int cvNlsResid_fused_Mi355(sunrealtype rl1, sunrealtype ngamma, N_Vector zn1, N_Vector ycor,
                            N_Vector ftemp, N_Vector res);
 
+/* No counterpart in the reference: the Newton iteration's update after the
+   linear solve as one kernel -- ycor = ycor + delta, y = zn0 + ycor, *dnrm the
+   WRMS norm of delta and, where cnrm is not NULL, *cnrm that of the new ycor
+   -- with the bits of the N_VLinearSum and N_VWrmsNorm calls.  -1, with
+   nothing done, for vectors that are not MI355X vectors of one stream and
+   length, or that add sequentially. */
+int cvNewtonUpdate_fused_Mi355(N_Vector delta, N_Vector ewt, N_Vector zn0, N_Vector ycor,
+                               N_Vector y, sunrealtype* dnrm, sunrealtype* cnrm);
+
 /* No counterpart in the reference (which fuses neither): the Nordsieck
    predictor and its undo of cvPredict / cvRestore (src/cvode/cvode.c:2748,
    2791) as one kernel over zn[0..q], q in 1..5 -- zn[j-1] = zn[j-1] +- zn[j]

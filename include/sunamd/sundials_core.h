@@ -169,6 +169,9 @@ SUNNonlinearSolver SUNNonlinSol_Newton(N_Vector y, SUNContext sunctx);
    the integrator's fused mode with the block LU's one-pass solve.
    SUN_ERR_ARG_INCOMPATIBLE for another solver type. */
 SUNErrCode SUNNonlinSol_NewtonSetNegatedLSolve(SUNNonlinearSolver NLS, sunbooleantype on);
+/* Likewise: the convergence test adds delta to ycor itself (the integrator's
+   fused mode updates and takes the norms in one pass). */
+SUNErrCode SUNNonlinSol_NewtonSetUpdateInConvTest(SUNNonlinearSolver NLS, sunbooleantype on);
 
 /* small math helpers with the reference's semantics (sundials_math.c:37-52,
    sundials_math.h:83,107,235) */

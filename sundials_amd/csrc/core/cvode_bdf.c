@@ -223,6 +223,10 @@ typedef struct CVodeMemRec
   int (*fused_lsetup)(SUNLinearSolver, SUNMatrix, SUNMatrix, sunrealtype, int);
   int (*fused_lsolve)(SUNLinearSolver, SUNMatrix, N_Vector, sunrealtype);
   sunbooleantype nls_negated; /* the Newton solver hands LSolve r, not -r */
+  /* ycor += delta, y = zn0 + ycor and both WRMS norms in one pass */
+  int (*fused_update)(N_Vector, N_Vector, N_Vector, N_Vector, N_Vector, sunrealtype*, sunrealtype*);
+  sunbooleantype nls_updates; /* the Newton solver leaves ycor += delta to the convergence test */
+  sunbooleantype y_current;   /* that test's pass has formed y for the present ycor */
 
   sunbooleantype MallocDone;
 } CVodeMemRec;
@@ -358,6 +362,7 @@ int CVodeSetNonlinearSolver(void* cvode_mem, SUNNonlinearSolver NLS)
   cv->NLS    = NLS;
   cv->ownNLS = SUNFALSE;
   cv->nls_negated = SUNFALSE; /* the new solver has not been told */
+  cv->nls_updates = SUNFALSE;
   if (SUNNonlinSolGetType(NLS) != SUNNONLINEARSOLVER_ROOTFIND) { return CV_ILL_INPUT; }
   if (SUNNonlinSolSetSysFn(NLS, cvNlsResidual) != SUN_SUCCESS) { return CV_ILL_INPUT; }
   if (SUNNonlinSolSetConvTestFn(NLS, cvNlsConvTest, cv) != SUN_SUCCESS)
@@ -580,6 +585,8 @@ int CVodeSetUseIntegratorFusedKernels(void* cvode_mem, sunbooleantype onoff)
                               int))dlsym(RTLD_DEFAULT, "SUNLinSol_Mi355BlockLUSetupScaled");
   cv->fused_lsolve = (int (*)(SUNLinearSolver, SUNMatrix, N_Vector,
                               sunrealtype))dlsym(RTLD_DEFAULT, "SUNLinSol_Mi355BlockLUSolveScaled");
+  cv->fused_update = (int (*)(N_Vector, N_Vector, N_Vector, N_Vector, N_Vector, sunrealtype*,
+                              sunrealtype*))dlsym(RTLD_DEFAULT, "cvNewtonUpdate_fused_Mi355");
   cv->usefused     = SUNTRUE;
   return CV_SUCCESS;
 }
@@ -890,8 +897,21 @@ static int cvNlsConvTest(SUNNonlinearSolver NLS, N_Vector ycor, N_Vector delta,
 {
   CVodeMem cv = (CVodeMem)mem;
   int m;
-  sunrealtype del = N_VWrmsNorm(delta, ewt);
   if (SUNNonlinSolGetCurIter(NLS, &m) != SUN_SUCCESS) { return CV_MEM_NULL; }
+  /* the norm of the whole correction, taken once the iteration has converged:
+     after one iteration from a zero start it is del (see below) */
+  const sunbooleantype cnrm_is_del = (m == 0 && !cv->nonzero_start);
+  sunrealtype del, cnrm = ZERO;
+  cv->y_current = SUNFALSE;
+  if (cv->nls_updates)
+  {
+    if (cv->fused_update(delta, ewt, cv->zn[0], ycor, cv->y, &del, cnrm_is_del ? NULL : &cnrm) == 0)
+    {
+      cv->y_current = SUNTRUE;
+    }
+    else { N_VLinearSum(ONE, ycor, ONE, delta, ycor); }
+  }
+  if (!cv->y_current) { del = N_VWrmsNorm(delta, ewt); }
   if (m > 0) { cv->crate = SUNMAX(CRDOWN * cv->crate, del / cv->delp); }
   sunrealtype dcon = del * SUNMIN(ONE, cv->crate) / tol;
   if (dcon <= ONE)
@@ -899,7 +919,7 @@ static int cvNlsConvTest(SUNNonlinearSolver NLS, N_Vector ycor, N_Vector delta,
     /* after one iteration from a zero start the correction is the update
        itself (the reference's shortcut); from a proposed start its norm has
        to be taken (after a restart from zero it equals del bit for bit) */
-    cv->acnrm    = (m == 0 && !cv->nonzero_start) ? del : N_VWrmsNorm(ycor, ewt);
+    cv->acnrm    = cnrm_is_del ? del : cv->y_current ? cnrm : N_VWrmsNorm(ycor, ewt);
     cv->acnrmcur = SUNTRUE;
     return CV_SUCCESS;
   }
@@ -911,7 +931,12 @@ static int cvNlsConvTest(SUNNonlinearSolver NLS, N_Vector ycor, N_Vector delta,
 static int cvNlsResidual(N_Vector ycor, N_Vector res, void* mem)
 {
   CVodeMem cv = (CVodeMem)mem;
-  N_VLinearSum(ONE, cv->zn[0], ONE, ycor, cv->y);
+  /* y stands from the convergence test's pass, unless the Newton solver has
+     started again from a cleared correction since (its count is zero then) */
+  int curiter = 0;
+  if (cv->y_current) { (void)SUNNonlinSolGetCurIter(cv->NLS, &curiter); }
+  if (curiter == 0) { N_VLinearSum(ONE, cv->zn[0], ONE, ycor, cv->y); }
+  cv->y_current = SUNFALSE;
   int retval = cv->f(cv->tn, cv->y, cv->ftemp, cv->user_data);
   cv->nfe++;
   if (retval < 0) { return CV_RHSFUNC_FAIL; }
@@ -1288,7 +1313,16 @@ static int cvNls(CVodeMem cv, int nflag)
                           ? neg
                           : SUNFALSE;
     }
+    /* likewise the update of the correction, into the convergence test */
+    const sunbooleantype upd = cv->usefused && cv->fused_update && cv->ownNLS;
+    if (upd != cv->nls_updates)
+    {
+      cv->nls_updates = (SUNNonlinSol_NewtonSetUpdateInConvTest(cv->NLS, upd) == SUN_SUCCESS)
+                          ? upd
+                          : SUNFALSE;
+    }
   }
+  cv->y_current = SUNFALSE;
   flag = SUNNonlinSolSolve(cv->NLS, cv->zn[0], cv->acor, cv->ewt, cv->tq[4],
                            callSetup, cv);
 
@@ -1299,7 +1333,7 @@ static int cvNls(CVodeMem cv, int nflag)
 
   if (flag != SUN_SUCCESS) { return flag; }
 
-  N_VLinearSum(ONE, cv->zn[0], ONE, cv->acor, cv->y);
+  if (!cv->y_current) { N_VLinearSum(ONE, cv->zn[0], ONE, cv->acor, cv->y); }
   if (!cv->acnrmcur) { cv->acnrm = N_VWrmsNorm(cv->acor, cv->ewt); }
   cv->jcur = SUNFALSE;
   return flag;

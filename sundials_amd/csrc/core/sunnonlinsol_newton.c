@@ -31,6 +31,7 @@ typedef struct
   long int nconvfails;
   void* ctest_data;
   sunbooleantype negated_lsolve; /* LSolve returns the solution for -b */
+  sunbooleantype ctest_updates;  /* CTest adds delta to ycor */
 } NewtonContent;
 
 #define NC(NLS) ((NewtonContent*)((NLS)->content))
@@ -89,7 +90,7 @@ static int newton_solve(SUNNonlinearSolver NLS, N_Vector y0, N_Vector ycor,
       retval = c->LSolve(delta, mem);
       if (retval != SUN_SUCCESS) { break; }
 
-      N_VLinearSum(SUN_RCONST(1.0), ycor, SUN_RCONST(1.0), delta, ycor);
+      if (!c->ctest_updates) { N_VLinearSum(SUN_RCONST(1.0), ycor, SUN_RCONST(1.0), delta, ycor); }
 
       retval = c->CTest(NLS, ycor, delta, tol, w, c->ctest_data);
       c->curiter++;
@@ -134,6 +135,16 @@ SUNErrCode SUNNonlinSol_NewtonSetNegatedLSolve(SUNNonlinearSolver NLS, sunboolea
 {
   if (!NLS || !NLS->content || NLS->ops->solve != newton_solve) { return SUN_ERR_ARG_INCOMPATIBLE; }
   NC(NLS)->negated_lsolve = on ? SUNTRUE : SUNFALSE;
+  return SUN_SUCCESS;
+}
+
+/* No counterpart in the reference.  With on, the convergence test is handed
+   ycor before the update and adds delta to it itself: for an integrator that
+   updates and takes its norms in one pass. */
+SUNErrCode SUNNonlinSol_NewtonSetUpdateInConvTest(SUNNonlinearSolver NLS, sunbooleantype on)
+{
+  if (!NLS || !NLS->content || NLS->ops->solve != newton_solve) { return SUN_ERR_ARG_INCOMPATIBLE; }
+  NC(NLS)->ctest_updates = on ? SUNTRUE : SUNFALSE;
   return SUN_SUCCESS;
 }
 

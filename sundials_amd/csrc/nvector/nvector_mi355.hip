@@ -47,7 +47,8 @@ typedef double dbl2 __attribute__((ext_vector_type(2)));
 // ----------------------------------------------------------------------------
 // execution context shared by a vector and all of its clones
 // ----------------------------------------------------------------------------
-#define NV_RESULT_SLOTS (NV_HOST_FOLD > NV_MAX_MULTI + 1 ? NV_HOST_FOLD : NV_MAX_MULTI + 1)
+#define NV_RESULT_SLOTS (2 * NV_HOST_FOLD) // two values per reduction at most (k_newton_update)
+static_assert(NV_RESULT_SLOTS >= NV_MAX_MULTI + 1, "the multi-vector results' slots");
 
 struct Mi355Exec
 {
@@ -380,7 +381,9 @@ __global__ void __launch_bounds__(NV_BLOCK) k_finish(const double* __restrict__ 
 // contiguous chunk); the last, partial chunk goes pair by pair.  Each lane
 // visits its pairs in increasing order, so per-lane accumulations have an
 // order fixed by np and the grid.
-template <int U, typename Load, typename Use>
+// With PIN the scheduler may not move those loads down among the uses, as it
+// does in a kernel of several inputs that also stores.
+template <int U, bool PIN = false, typename Load, typename Use>
 __device__ __forceinline__ void chunk_pairs(long np, Load load, Use use)
 {
   const long chunk = (long)U * NV_BLOCK;
@@ -392,6 +395,7 @@ __device__ __forceinline__ void chunk_pairs(long np, Load load, Use use)
       decltype(load(0L)) v[U];
 #pragma unroll
       for (int u = 0; u < U; u++) { v[u] = load(i0 + (long)u * NV_BLOCK); }
+      if constexpr (PIN) { __builtin_amdgcn_sched_barrier(0); }
 #pragma unroll
       for (int u = 0; u < U; u++) { use(i0 + (long)u * NV_BLOCK, v[u]); }
     }
@@ -1888,6 +1892,100 @@ extern "C" SUNErrCode SUNAMD_ClassicalGS_Mi355(N_Vector* v, sunrealtype** h, int
     *new_vk_norm = (nn <= 0.0) ? 0.0 : sqrt(nn);
   }
   return SUN_SUCCESS;
+}
+
+// ----------------------------------------------------------------------------
+// CVODE's Newton iteration after the linear solve (cvode_nls.c:269-320 and
+// sunnonlinsol_newton.c:252-255), in its fused mode: ycor += delta, y = zn0 +
+// ycor and the WRMS norms of delta and of the new ycor, in one pass.
+// What bounds it: launches at the sizes one system has (2^14 cells x 32
+// species: two LinearSums of 4.5 us, a norm of 4.0 us and, for every iteration
+// after the first, another norm with its wait -> one kernel of 6.5 us; 9.0 us
+// with the loads left to the scheduler), HBM beyond (64 or 80 -> 48 bytes per
+// element).  The lanes' pairs, the workgroups and the fold are
+// k_reduce<RK_WSQR>'s, so the norms have its bits, at any n.
+// ----------------------------------------------------------------------------
+template <int NV>
+__global__ void __launch_bounds__(NV_BLOCK)
+  k_newton_update(const double* __restrict__ delta, const double* __restrict__ ewt,
+                  const double* __restrict__ zn0, double* __restrict__ ycor,
+                  double* __restrict__ y, long n, double* partials, int to_host)
+{
+  double acc[NV];
+#pragma unroll
+  for (int k = 0; k < NV; k++) { acc[k] = 0.0; }
+  auto add = [&](double d, double w, double c) {
+    acc[0] = acc[0] + red_elem<RK_WSQR>(d, w, 0.0);
+    if (NV == 2) { acc[NV - 1] = acc[NV - 1] + red_elem<RK_WSQR>(c, w, 0.0); }
+  };
+  chunk_pairs<unroll_for(red_loads<RK_WSQR>()), true>(
+    n >> 1, [&](long i) { return Pairs<4>{{ld2(delta, i), ld2(ewt, i), ld2(zn0, i), ld2(ycor, i)}}; },
+    [&](long i, const Pairs<4>& p) {
+      const dbl2 c = p.v[3] + p.v[0];
+      st2(ycor, i, c);
+      st2(y, i, p.v[2] + c);
+      add(p.v[0].x, p.v[1].x, c.x);
+      add(p.v[0].y, p.v[1].y, c.y);
+    });
+  TAIL(n)
+  {
+    const double c = ycor[n - 1] + delta[n - 1];
+    ycor[n - 1]    = c;
+    y[n - 1]       = zn0[n - 1] + c;
+    add(delta[n - 1], ewt[n - 1], c);
+  }
+  grid_finish<RSUM, NV>(acc, partials, to_host);
+}
+
+// *cnrm is computed where cnrm is not NULL.  -1, with nothing done: a vector of
+// another kind, stream or length, or one whose sums run in sequential order.
+extern "C" int cvNewtonUpdate_fused_Mi355(N_Vector delta, N_Vector ewt, N_Vector zn0, N_Vector ycor,
+                                          N_Vector y, sunrealtype* dnrm, sunrealtype* cnrm)
+{
+  const N_Vector all[5] = {delta, ewt, zn0, ycor, y};
+  for (int i = 0; i < 5; i++)
+  {
+    if (!SUNAMD_NVectorIsMi355(all[i]) || EXEC(all[i]) != EXEC(delta) ||
+        NVLEN(all[i]) != NVLEN(delta))
+    {
+      return -1;
+    }
+  }
+  if (CONTENT(delta)->red_order == SUNAMD_REDUCE_SEQUENTIAL ||
+      CONTENT(ycor)->red_order == SUNAMD_REDUCE_SEQUENTIAL)
+  {
+    return -1;
+  }
+  const long n  = (long)NVLEN(delta);
+  Mi355Exec* ex = EXEC(delta);
+  if (n == 0 || DDATA(y) == DDATA(ycor) || DDATA(y) == DDATA(zn0) || DDATA(y) == DDATA(delta) ||
+      DDATA(y) == DDATA(ewt))
+  {
+    return -1;
+  }
+  const int nv    = cnrm ? 2 : 1;
+  const int g     = red_grid(ex, n >> 1, unroll_for(red_loads<RK_WSQR>()));
+  const int fold  = g <= NV_HOST_FOLD;
+  const int slots = fold ? nv * g : nv;
+  slots_clear(ex, slots);
+  sunamd_prof_begin(SUNAMD_K_WRMS, ex->stream);
+  auto kern = cnrm ? k_newton_update<2> : k_newton_update<1>;
+  kern<<<g, NV_BLOCK, 0, ex->stream>>>(DDATA(delta), DDATA(ewt), DDATA(zn0), DDATA(ycor), DDATA(y),
+                                       n, fold ? ex->h_result : ex->d_partials, fold);
+  if (!fold)
+  {
+    k_finish<RSUM><<<nv, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->h_result, 0.0);
+  }
+  sunamd_prof_end(SUNAMD_K_WRMS, ex->stream);
+  LAUNCHCHK(delta);
+  HIPCHK_EX(delta, slots_wait(ex, slots));
+  sunrealtype* out[2] = {dnrm, cnrm};
+  for (int k = 0; k < nv; k++)
+  {
+    const double ss = fold ? fold_on_host<RSUM>(ex->h_result + k * g, g, 0.0) : ex->h_result[k];
+    *out[k]         = ex->err != hipSuccess ? NAN : sqrt0(ss / (double)n);
+  }
+  return 0;
 }
 
 extern "C" int N_VGetHipError_Mi355(N_Vector v)

@@ -107,3 +107,28 @@ def test_gram_schmidt_passes(ctx, k):
     assert abs(norm.value / np.linalg.norm(z) - 1) <= n * 2.0 ** -53
     for v in vs + tmp:
         core.N_VDestroy(v)
+
+
+@pytest.mark.parametrize("with_cnrm", [False, True])
+@pytest.mark.parametrize("n", EDGES)
+def test_newton_update_equals_the_single_ops(ctx, n, with_cnrm):
+    core, fn = _lib.core(), _lib.hip().cvNewtonUpdate_fused_Mi355
+    fn.restype, fn.argtypes = C.c_int, [C.c_void_p] * 5 + [C.POINTER(C.c_double)] * 2
+    rng = np.random.default_rng(n)
+    d, z, c = (rng.standard_normal(n) for _ in range(3))
+    w = rng.uniform(0.5, 2, n)
+    vd, vw, vz, vc, vy, ref_y = (gpu_vec(ctx, a) for a in (d, w, z, c, np.zeros(n), np.zeros(n)))
+    dn, cn = C.c_double(-1.0), C.c_double(-1.0)
+    assert fn(vd, vw, vz, vc, vy, C.byref(dn), C.byref(cn) if with_cnrm else None) == 0
+    ref_c = gpu_vec(ctx, c)
+    core.N_VLinearSum(1.0, ref_c, 1.0, vd, ref_c)
+    core.N_VLinearSum(1.0, vz, 1.0, ref_c, ref_y)
+    assert np.array_equal(gpu_get(vc), gpu_get(ref_c)) and np.array_equal(gpu_get(vy), gpu_get(ref_y))
+    assert dn.value == core.N_VWrmsNorm(vd, vw)
+    assert cn.value == (core.N_VWrmsNorm(ref_c, vw) if with_cnrm else -1.0)
+    short = gpu_vec(ctx, np.zeros(n + 1))
+    assert fn(vd, vw, vz, vc, short, C.byref(dn), None) == -1  # another length: nothing done
+    assert fn(vd, vw, vz, vc, vz, C.byref(dn), None) == -1     # y is zn0
+    assert np.array_equal(gpu_get(vc), gpu_get(ref_c))
+    for v in (vd, vw, vz, vc, vy, ref_y, ref_c, short):
+        core.N_VDestroy(v)
