@@ -123,6 +123,9 @@ int cvNewtonUpdate_fused_Mi355(N_Vector delta, N_Vector ewt, N_Vector zn0, N_Vec
    CVodeSetUseIntegratorFusedKernels; -1 for vectors that are not MI355X
    vectors. */
 int cvPredict_fused_Mi355(int q, N_Vector* zn);
+/* the predictor and, in the same pass, acor = 0 and y = zn[0] + 0; -1, with
+   nothing done, where acor or y is of another kind, stream or length */
+int cvPredictStart_fused_Mi355(int q, N_Vector* zn, N_Vector acor, N_Vector y);
 int cvRestore_fused_Mi355(int q, N_Vector* zn);
 
 /* No counterpart in the reference (KINSOL has no fused kernels): KINSOL's

@@ -218,6 +218,9 @@ typedef struct CVodeMemRec
   int (*fused_resid)(sunrealtype, sunrealtype, N_Vector, N_Vector, N_Vector, N_Vector);
   int (*fused_predict)(int, N_Vector*); /* Nordsieck predictor / its undo in one pass */
   int (*fused_restore)(int, N_Vector*);
+  /* the predictor with acor = 0 and y = zn0 + 0 */
+  int (*fused_predict_start)(int, N_Vector*, N_Vector, N_Vector);
+  sunbooleantype started; /* that pass has run for the coming Newton iteration */
   /* copy + ScaleAddI + factorisation of the Newton matrix in one pass (NULL:
      the library has none); declines with SUN_ERR_ARG_INCOMPATIBLE */
   int (*fused_lsetup)(SUNLinearSolver, SUNMatrix, SUNMatrix, sunrealtype, int);
@@ -587,6 +590,8 @@ int CVodeSetUseIntegratorFusedKernels(void* cvode_mem, sunbooleantype onoff)
                               sunrealtype))dlsym(RTLD_DEFAULT, "SUNLinSol_Mi355BlockLUSolveScaled");
   cv->fused_update = (int (*)(N_Vector, N_Vector, N_Vector, N_Vector, N_Vector, sunrealtype*,
                               sunrealtype*))dlsym(RTLD_DEFAULT, "cvNewtonUpdate_fused_Mi355");
+  cv->fused_predict_start =
+    (int (*)(int, N_Vector*, N_Vector, N_Vector))dlsym(RTLD_DEFAULT, "cvPredictStart_fused_Mi355");
   cv->usefused     = SUNTRUE;
   return CV_SUCCESS;
 }
@@ -931,11 +936,13 @@ static int cvNlsConvTest(SUNNonlinearSolver NLS, N_Vector ycor, N_Vector delta,
 static int cvNlsResidual(N_Vector ycor, N_Vector res, void* mem)
 {
   CVodeMem cv = (CVodeMem)mem;
-  /* y stands from the convergence test's pass, unless the Newton solver has
-     started again from a cleared correction since (its count is zero then) */
+  /* y stands from the predictor's pass at the first residual, and from the
+     convergence test's pass unless the Newton solver has started again from a
+     cleared correction since (its count is zero then) */
   int curiter = 0;
   if (cv->y_current) { (void)SUNNonlinSolGetCurIter(cv->NLS, &curiter); }
-  if (curiter == 0) { N_VLinearSum(ONE, cv->zn[0], ONE, ycor, cv->y); }
+  if (!cv->started && curiter == 0) { N_VLinearSum(ONE, cv->zn[0], ONE, ycor, cv->y); }
+  cv->started   = SUNFALSE;
   cv->y_current = SUNFALSE;
   int retval = cv->f(cv->tn, cv->y, cv->ftemp, cv->user_data);
   cv->nfe++;
@@ -1187,6 +1194,11 @@ static void cvPredict(CVodeMem cv)
   {
     if ((cv->tn - cv->tstop) * cv->h > ZERO) { cv->tn = cv->tstop; }
   }
+  /* with the integrator's own Newton solver, whose first residual is that of
+     the zero correction, the same pass clears acor and forms y */
+  cv->started = cv->usefused && cv->fused_predict_start && cv->ownNLS &&
+                cv->fused_predict_start(cv->q, cv->zn, cv->acor, cv->y) == 0;
+  if (cv->started) { return; }
   if (cv->usefused && cv->fused_predict(cv->q, cv->zn) == 0) { return; }
   for (int k = 1; k <= cv->q; k++)
   {
@@ -1283,7 +1295,7 @@ static int cvNls(CVodeMem cv, int nflag)
   }
 
   /* initial guess for the correction: zero, or the caller's proposal */
-  N_VConst(ZERO, cv->acor);
+  if (!cv->started) { N_VConst(ZERO, cv->acor); }
   cv->nonzero_start = SUNFALSE;
   if (cv->initcor)
   {
@@ -1291,6 +1303,7 @@ static int cvNls(CVodeMem cv, int nflag)
     {
       cv->ninit_used++;
       cv->nonzero_start = SUNTRUE;
+      cv->started       = SUNFALSE;
     }
     else { N_VConst(ZERO, cv->acor); }
   }

@@ -132,3 +132,29 @@ def test_newton_update_equals_the_single_ops(ctx, n, with_cnrm):
     assert np.array_equal(gpu_get(vc), gpu_get(ref_c))
     for v in (vd, vw, vz, vc, vy, ref_y, ref_c, short):
         core.N_VDestroy(v)
+
+
+@pytest.mark.parametrize("q", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("n", [1, 2, 2047, 2048, 2051, 300001])
+def test_predictor_with_the_newton_start(ctx, n, q):
+    core, hip = _lib.core(), _lib.hip()
+    plain, start = hip.cvPredict_fused_Mi355, hip.cvPredictStart_fused_Mi355
+    plain.restype = start.restype = C.c_int
+    rng = np.random.default_rng(n + q)
+    z = rng.standard_normal((q + 1, n))
+    z[0, -1], z[1:, -1] = -0.0, -0.0  # -0 + 0 is +0 in y, and stays -0 in zn
+    a, b = ([gpu_vec(ctx, r) for r in z] for _ in range(2))
+    acor, y, ref = (gpu_vec(ctx, rng.standard_normal(n)) for _ in range(3))
+    zero = gpu_vec(ctx, np.zeros(n))
+    assert plain(q, vec_array(a)) == 0
+    core.N_VLinearSum(1.0, a[0], 1.0, zero, ref)
+    assert start(q, vec_array(b), C.c_void_p(acor), C.c_void_p(y)) == 0
+    bits = lambda v: gpu_get(v).view(np.int64)  # noqa: E731
+    assert all(np.array_equal(bits(u), bits(v)) for u, v in zip(a, b))
+    assert np.array_equal(bits(y), bits(ref)) and not bits(acor).any()
+    short = gpu_vec(ctx, np.zeros(n + 1))
+    for bad in ((acor, short), (b[1], y), (acor, b[0]), (y, y)):
+        assert start(q, vec_array(b), *map(C.c_void_p, bad)) == -1
+    assert all(np.array_equal(bits(u), bits(v)) for u, v in zip(a, b))
+    for v in (*a, *b, acor, y, ref, zero, short):
+        core.N_VDestroy(v)
