@@ -53,59 +53,11 @@ __device__ __forceinline__ float readlane_d(float x, int l)
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
 }
 
-// ---- pivot search: largest |a_ik| over the group, ties to the smallest row
-// (the dense GETRF's first maximum), as a reduction on (value, row) pairs:
-// DPP exchanges inside rows of 16 lanes, lane reads across rows --------------
-
-// (ov, op) replaces (v, p) when ov is larger, or equal with a smaller row;
-// evaluated without short-circuit so it compiles to compares and selects
-template <typename V>
-__device__ __forceinline__ void amax_take(V& v, int& p, V ov, int op)
-{
-  const bool take = (ov > v) | ((ov == v) & (op < p));
-  v               = take ? ov : v;
-  p               = take ? op : p;
-}
-
-template <int CTRL, typename V>
-__device__ __forceinline__ void amax_dpp(V& v, int& p)
-{
-  const V ov   = dpp_v<CTRL>(v);
-  const int op = dpp_i<CTRL>(p);
-  amax_take(v, p, ov, op);
-}
-
-// every lane of a G-lane group (G a power of two, groups aligned to G lanes)
-// ends with the group's maximum pair
-template <int G, typename V>
-__device__ __forceinline__ void g_argmax(V& v, int& p)
-{
-  if constexpr (G >= 2) { amax_dpp<0xB1>(v, p); }  // quad_perm [1,0,3,2]
-  if constexpr (G >= 4) { amax_dpp<0x4E>(v, p); }  // quad_perm [2,3,0,1]
-  if constexpr (G >= 8) { amax_dpp<0x141>(v, p); } // row_half_mirror
-  if constexpr (G >= 16) { amax_dpp<0x140>(v, p); } // row_mirror
-  if constexpr (G >= 32)
-  {
-    const V r0 = readlane_d(v, 0), r1 = readlane_d(v, 16);
-    const V r2 = readlane_d(v, 32), r3 = readlane_d(v, 48);
-    const int p0 = __builtin_amdgcn_readlane(p, 0), p1 = __builtin_amdgcn_readlane(p, 16);
-    const int p2 = __builtin_amdgcn_readlane(p, 32), p3 = __builtin_amdgcn_readlane(p, 48);
-    V a = r0, b = r2;
-    int pa = p0, pb = p2;
-    amax_take(a, pa, r1, p1);
-    amax_take(b, pb, r3, p3);
-    if constexpr (G == 64) { amax_take(a, pa, b, pb); }
-    const bool hi_half = (G == 32) && (__lane_id() >= 32);
-    v = hi_half ? b : a;
-    p = hi_half ? pb : pa;
-  }
-}
-
 // ---- pivot search of the double- and single-precision factorisations -------
 // The dense GETRF's choice (sundials_dense.c:94-100): the largest |a_ik| over
-// the rows at positions >= k, the first one on ties.  g_argmax carries a
-// (value, position) pair through every exchange (about 75 VALU instructions
-// per column in FP64); here the exchanges carry one 32-bit word, the value's
+// the rows at positions >= k, the first one on ties.  A (value, position) pair
+// carried through every exchange takes about 75 VALU instructions per column
+// in FP64; here the exchanges carry one 32-bit word, the value's
 // high half, as an unsigned maximum (a DPP v_max_u32 per level), and the
 // lanes that hold that maximum are counted with a ballot.  One holder is the
 // pivot.  Several holders (a tie in the high half, all zero) are told apart by
