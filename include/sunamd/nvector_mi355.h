@@ -123,6 +123,10 @@ int cvNewtonUpdate_fused_Mi355(N_Vector delta, N_Vector ewt, N_Vector zn0, N_Vec
    CVodeSetUseIntegratorFusedKernels; -1 for vectors that are not MI355X
    vectors. */
 int cvPredict_fused_Mi355(int q, N_Vector* zn);
+/* cvEwtSetSS_fused_Mi355 and, in the same pass, *nrm = N_VWrmsNorm(ycur, weight)
+   bit for bit; -1, with nothing done, as cvNewtonUpdate_fused_Mi355 */
+int cvEwtSetSSNorm_fused_Mi355(sunrealtype reltol, sunrealtype Sabstol, N_Vector ycur,
+                               N_Vector tempv, N_Vector weight, sunrealtype* nrm);
 /* the predictor and, in the same pass, acor = 0 and y = zn[0] + 0; -1, with
    nothing done, where acor or y is of another kind, stream or length */
 int cvPredictStart_fused_Mi355(int q, N_Vector* zn, N_Vector acor, N_Vector y);

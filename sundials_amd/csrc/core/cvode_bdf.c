@@ -218,6 +218,8 @@ typedef struct CVodeMemRec
   int (*fused_resid)(sunrealtype, sunrealtype, N_Vector, N_Vector, N_Vector, N_Vector);
   int (*fused_predict)(int, N_Vector*); /* Nordsieck predictor / its undo in one pass */
   int (*fused_restore)(int, N_Vector*);
+  /* error weights for scalar tolerances with the norm of the state under them */
+  int (*fused_ewt_norm)(sunrealtype, sunrealtype, N_Vector, N_Vector, N_Vector, sunrealtype*);
   /* the predictor with acor = 0 and y = zn0 + 0 */
   int (*fused_predict_start)(int, N_Vector*, N_Vector, N_Vector);
   sunbooleantype started; /* that pass has run for the coming Newton iteration */
@@ -590,6 +592,8 @@ int CVodeSetUseIntegratorFusedKernels(void* cvode_mem, sunbooleantype onoff)
                               sunrealtype))dlsym(RTLD_DEFAULT, "SUNLinSol_Mi355BlockLUSolveScaled");
   cv->fused_update = (int (*)(N_Vector, N_Vector, N_Vector, N_Vector, N_Vector, sunrealtype*,
                               sunrealtype*))dlsym(RTLD_DEFAULT, "cvNewtonUpdate_fused_Mi355");
+  cv->fused_ewt_norm = (int (*)(sunrealtype, sunrealtype, N_Vector, N_Vector, N_Vector,
+                                sunrealtype*))dlsym(RTLD_DEFAULT, "cvEwtSetSSNorm_fused_Mi355");
   cv->fused_predict_start =
     (int (*)(int, N_Vector*, N_Vector, N_Vector))dlsym(RTLD_DEFAULT, "cvPredictStart_fused_Mi355");
   cv->usefused     = SUNTRUE;
@@ -1736,9 +1740,15 @@ int CVode(void* cvode_mem, sunrealtype tout, N_Vector yout, sunrealtype* tret, i
     cv->next_h = cv->h;
     cv->next_q = cv->q;
 
+    sunbooleantype have_nrm = SUNFALSE;
     if (cv->nst > 0)
     {
-      if (cvEwtSet(cv->zn[0], cv->ewt, cv) != 0)
+      /* with scalar tolerances that need no component test, the weights'
+         pass also takes the norm below */
+      have_nrm = cv->usefused && cv->fused_ewt_norm && cv->itol == CV_SS && !cv->atolmin0 &&
+                 cv->fused_ewt_norm(cv->reltol, cv->Sabstol, cv->zn[0], cv->tempv, cv->ewt,
+                                    &nrm) == 0;
+      if (!have_nrm && cvEwtSet(cv->zn[0], cv->ewt, cv) != 0)
       {
         istate       = CV_ILL_INPUT;
         cv->tretlast = *tret = cv->tn;
@@ -1755,7 +1765,7 @@ int CVode(void* cvode_mem, sunrealtype tout, N_Vector yout, sunrealtype* tret, i
       break;
     }
 
-    nrm       = N_VWrmsNorm(cv->zn[0], cv->ewt);
+    if (!have_nrm) { nrm = N_VWrmsNorm(cv->zn[0], cv->ewt); }
     cv->tolsf = cv->uround * nrm;
     if (cv->tolsf > ONE)
     {

@@ -27,6 +27,7 @@
 
 #include <cmath>
 #include <cstdio>
+#include <initializer_list>
 #include <cstdlib>
 #include <cstring>
 #include <ctime>
@@ -1985,6 +1986,79 @@ extern "C" int cvNewtonUpdate_fused_Mi355(N_Vector delta, N_Vector ewt, N_Vector
     const double ss = fold ? fold_on_host<RSUM>(ex->h_result + k * g, g, 0.0) : ex->h_result[k];
     *out[k]         = ex->err != hipSuccess ? NAN : sqrt0(ss / (double)n);
   }
+  return 0;
+}
+
+// ----------------------------------------------------------------------------
+// The start of a CVODE step in its fused mode: the error weights for scalar
+// tolerances (k_ewt_ss's sequence) and the WRMS norm of the state under them,
+// one pass and one launch instead of two (2^14 cells x 32 species: 4.4 + 4.0
+// -> 5.7 us; 40 -> 24 bytes per element).  Pairs and fold as k_newton_update's.
+// ----------------------------------------------------------------------------
+__global__ void __launch_bounds__(NV_BLOCK)
+  k_ewt_norm(double rtol, double atol, const double* __restrict__ x, double* __restrict__ tempv,
+             double* __restrict__ w, long n, double* partials, int to_host)
+{
+  double acc[1] = {0.0};
+  chunk_pairs<unroll_for(red_loads<RK_WSQR>()), true>(
+    n >> 1, [&](long i) { return Pairs<1>{{ld2(x, i)}}; },
+    [&](long i, const Pairs<1>& p) {
+      dbl2 t, v;
+      t.x = rtol * fabs(p.v[0].x);
+      t.y = rtol * fabs(p.v[0].y);
+      t.x = t.x + atol;
+      t.y = t.y + atol;
+      v.x = 1.0 / t.x;
+      v.y = 1.0 / t.y;
+      st2(tempv, i, t);
+      st2(w, i, v);
+      acc[0] = acc[0] + red_elem<RK_WSQR>(p.v[0].x, v.x, 0.0);
+      acc[0] = acc[0] + red_elem<RK_WSQR>(p.v[0].y, v.y, 0.0);
+    });
+  TAIL(n)
+  {
+    const double t = rtol * fabs(x[n - 1]) + atol;
+    const double v = 1.0 / t;
+    tempv[n - 1]   = t;
+    w[n - 1]       = v;
+    acc[0]         = acc[0] + red_elem<RK_WSQR>(x[n - 1], v, 0.0);
+  }
+  grid_finish<RSUM, 1>(acc, partials, to_host);
+}
+
+// -1, with nothing done: vectors of another kind, stream or length, sequential
+// sums, or outputs that are the input
+extern "C" int cvEwtSetSSNorm_fused_Mi355(sunrealtype reltol, sunrealtype Sabstol, N_Vector ycur,
+                                          N_Vector tempv, N_Vector weight, sunrealtype* nrm)
+{
+  for (N_Vector v : {ycur, tempv, weight})
+  {
+    if (!SUNAMD_NVectorIsMi355(v) || EXEC(v) != EXEC(ycur) || NVLEN(v) != NVLEN(ycur)) { return -1; }
+  }
+  const long n  = (long)NVLEN(ycur);
+  Mi355Exec* ex = EXEC(ycur);
+  if (n == 0 || CONTENT(ycur)->red_order == SUNAMD_REDUCE_SEQUENTIAL ||
+      DDATA(tempv) == DDATA(ycur) || DDATA(weight) == DDATA(ycur) || DDATA(tempv) == DDATA(weight))
+  {
+    return -1;
+  }
+  const int g     = red_grid(ex, n >> 1, unroll_for(red_loads<RK_WSQR>()));
+  const int fold  = g <= NV_HOST_FOLD;
+  const int slots = fold ? g : 1;
+  slots_clear(ex, slots);
+  sunamd_prof_begin(SUNAMD_K_WRMS, ex->stream);
+  k_ewt_norm<<<g, NV_BLOCK, 0, ex->stream>>>(reltol, Sabstol, DDATA(ycur), DDATA(tempv),
+                                             DDATA(weight), n, fold ? ex->h_result : ex->d_partials,
+                                             fold);
+  if (!fold)
+  {
+    k_finish<RSUM><<<1, NV_BLOCK, 0, ex->stream>>>(ex->d_partials, g, ex->h_result, 0.0);
+  }
+  sunamd_prof_end(SUNAMD_K_WRMS, ex->stream);
+  LAUNCHCHK(ycur);
+  HIPCHK_EX(ycur, slots_wait(ex, slots));
+  const double ss = fold ? fold_on_host<RSUM>(ex->h_result, g, 0.0) : ex->h_result[0];
+  *nrm            = ex->err != hipSuccess ? NAN : sqrt0(ss / (double)n);
   return 0;
 }
 

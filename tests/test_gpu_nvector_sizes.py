@@ -158,3 +158,20 @@ def test_predictor_with_the_newton_start(ctx, n, q):
     assert all(np.array_equal(bits(u), bits(v)) for u, v in zip(a, b))
     for v in (*a, *b, acor, y, ref, zero, short):
         core.N_VDestroy(v)
+
+
+@pytest.mark.parametrize("n", EDGES)
+def test_error_weights_with_the_norm(ctx, n):
+    core, fn = _lib.core(), _lib.hip().cvEwtSetSSNorm_fused_Mi355
+    fn.restype = C.c_int
+    fn.argtypes = [C.c_double] * 2 + [C.c_void_p] * 3 + [C.POINTER(C.c_double)]
+    x = np.random.default_rng(n).standard_normal(n)
+    vx, vt, vw = (gpu_vec(ctx, a) for a in (x, np.zeros(n), np.zeros(n)))
+    nrm = C.c_double(-1.0)
+    assert fn(1e-5, 1e-9, vx, vt, vw, C.byref(nrm)) == 0
+    t = 1e-5 * np.abs(x) + 1e-9
+    assert np.array_equal(gpu_get(vt), t) and np.array_equal(gpu_get(vw), 1.0 / t)
+    assert nrm.value == core.N_VWrmsNorm(vx, vw)
+    assert fn(1e-5, 1e-9, vx, vx, vw, C.byref(nrm)) == -1
+    for v in (vx, vt, vw):
+        core.N_VDestroy(v)
