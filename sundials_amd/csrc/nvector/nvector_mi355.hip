@@ -985,7 +985,9 @@ static constexpr double SLOT_WAIT_S            = 2e-3;
 // Every so many results the stream is synchronised all the same: the runtime
 // retires finished launches there, and a backlog of them (thousands, after
 // some hundred steps) would be retired at the caller's next synchronising call
-// instead.  It costs each result 1/SLOT_SYNC_EVERY of a synchronisation.
+// instead.  It costs each result 1/SLOT_SYNC_EVERY of a synchronisation (every
+// 8 results: a BDF step's ops on 32768 elements 72 -> 82 us, a coupled
+// integration of 2^14 x 32 189 -> 200 ms).
 static constexpr int SLOT_SYNC_EVERY = 32;
 
 static inline void slots_clear(Mi355Exec* ex, int count)
