@@ -21,6 +21,7 @@
 #include <cstring>
 
 #include "../core/profiler_internal.h"
+#include "block_place.h"
 #include "blocklu.h"
 #include "sunamd/nvector_mi355.h"
 #include "sunamd/sunamd_profiler.h"
@@ -66,10 +67,11 @@ __global__ void k_fill(double* __restrict__ a, long n, double v)
 }
 
 // A = c*A + I (per element: a *= c; a += 1 on the diagonal), HBM-bound.  A
-// thread takes pairs of elements and carries its place in the block along (the
-// stride's remainder added, one conditional subtraction) instead of a 64-bit
-// division per element: m = 21, 50000 blocks (353 MB) 60 -> 53 us.  U: unsigned
-// while m*m fits in it.
+// thread takes pairs of elements, finds its first pair's place in its block by
+// one 64-bit division and tests for the diagonal in U (unsigned while m*m fits
+// in it), where every element took a 64-bit division of its own: m = 21, 50000
+// blocks (353 MB, one pair per thread) 60 -> 53 us.  Beyond 2^25 elements, where
+// a thread takes several pairs, the place is carried along the stride.
 template <typename U>
 __global__ void __launch_bounds__(EW_BLOCK) k_scaleaddi(double* __restrict__ a, long n, long m,
                                                         double c)
@@ -98,8 +100,7 @@ __global__ void __launch_bounds__(EW_BLOCK) k_scaleaddi(double* __restrict__ a, 
       if (at % m1 == 0) { v = v + 1.0; }
       a[i] = v;
     }
-    at += by;
-    if (at >= mm) { at -= mm; }
+    at = block_place_after<U>(at, by, mm);
   }
 }
 

@@ -112,3 +112,22 @@ def test_every_size_follows_the_dense_solver(ctx, m, prec):
         r = b[k].copy()
         orc.oracle_block_getrs(dp(o), m, p.ctypes.data_as(C.POINTER(C.c_int64)), dp(r))
         assert np.array_equal(x[k], r, equal_nan=not finite), ("solve", k)
+
+
+def test_scale_add_i_over_several_pairs_per_thread(ctx):
+    """Beyond 2^25 elements a thread takes a pair, then the one a whole grid
+    further, at another place of its block (2^25 mod 441 = 65); the total is
+    odd, so the last element stands alone."""
+    core, hip = _lib.core(), _lib.hip()
+    nb, m, c = 80001, 21, -0.3125
+    y = gpu_vec(ctx, np.zeros(1))
+    M = hip.SUNMatrix_Mi355BlockDense(nb, m, hip.N_VGetStream_Mi355(y), ctx)
+    a = np.random.default_rng(21).uniform(-1, 1, nb * m * m)
+    C.memmove(hip.SUNMatrix_Mi355BlockDense_HostData(M), dp(a), 8 * a.size)
+    assert hip.SUNMatrix_Mi355BlockDense_CopyToDevice(M) == 0
+    assert core.SUNMatScaleAddI(c, M) == 0
+    a *= c
+    a.reshape(nb, m * m)[:, ::m + 1] += 1.0
+    assert np.array_equal(_gpu_matrix_values(hip, M, nb, m), a)
+    core.SUNMatDestroy(M)
+    core.N_VDestroy(y)
