@@ -111,7 +111,8 @@ int cvNlsResid_fused_Mi355(sunrealtype rl1, sunrealtype ngamma, N_Vector zn1, N_
    WRMS norm of delta and, where cnrm is not NULL, *cnrm that of the new ycor
    -- with the bits of the N_VLinearSum and N_VWrmsNorm calls.  -1, with
    nothing done, for vectors that are not MI355X vectors of one stream and
-   length, or that add sequentially. */
+   length, or that add sequentially, or where ycor or y shares its data with
+   another of the five. */
 int cvNewtonUpdate_fused_Mi355(N_Vector delta, N_Vector ewt, N_Vector zn0, N_Vector ycor,
                                N_Vector y, sunrealtype* dnrm, sunrealtype* cnrm);
 

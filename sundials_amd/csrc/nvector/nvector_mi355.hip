@@ -1941,7 +1941,8 @@ __global__ void __launch_bounds__(NV_BLOCK)
 }
 
 // *cnrm is computed where cnrm is not NULL.  -1, with nothing done: a vector of
-// another kind, stream or length, or one whose sums run in sequential order.
+// another kind, stream or length, one whose sums run in sequential order, or
+// ycor or y sharing its data with another of the five.
 extern "C" int cvNewtonUpdate_fused_Mi355(N_Vector delta, N_Vector ewt, N_Vector zn0, N_Vector ycor,
                                           N_Vector y, sunrealtype* dnrm, sunrealtype* cnrm)
 {
@@ -1961,11 +1962,14 @@ extern "C" int cvNewtonUpdate_fused_Mi355(N_Vector delta, N_Vector ewt, N_Vector
   }
   const long n  = (long)NVLEN(delta);
   Mi355Exec* ex = EXEC(delta);
-  if (n == 0 || DDATA(y) == DDATA(ycor) || DDATA(y) == DDATA(zn0) || DDATA(y) == DDATA(delta) ||
-      DDATA(y) == DDATA(ewt))
+  if (n == 0) { return -1; }
+  // an output that is another of the vectors would change what the separate
+  // calls read after it is written
+  for (N_Vector in : {delta, ewt, zn0})
   {
-    return -1;
+    if (DDATA(in) == DDATA(ycor) || DDATA(in) == DDATA(y)) { return -1; }
   }
+  if (DDATA(y) == DDATA(ycor)) { return -1; }
   const int nv    = cnrm ? 2 : 1;
   const int g     = red_grid(ex, n >> 1, unroll_for(red_loads<RK_WSQR>()));
   const int fold  = g <= NV_HOST_FOLD;

@@ -175,3 +175,24 @@ def test_error_weights_with_the_norm(ctx, n):
     assert fn(1e-5, 1e-9, vx, vx, vw, C.byref(nrm)) == -1
     for v in (vx, vt, vw):
         core.N_VDestroy(v)
+
+
+@pytest.mark.parametrize("shared", ["ycor=delta", "ycor=ewt", "ycor=zn0", "y=delta", "y=ewt", "y=zn0",
+                                    "y=ycor"])
+def test_newton_update_declines_shared_outputs(ctx, shared):
+    """N_VLinearSum into a vector that a later call of the sequence reads gives
+    other values than one pass: such calls are declined and touch nothing."""
+    core, fn = _lib.core(), _lib.hip().cvNewtonUpdate_fused_Mi355
+    fn.restype, fn.argtypes = C.c_int, [C.c_void_p] * 5 + [C.POINTER(C.c_double)] * 2
+    n = 1001
+    names = ("delta", "ewt", "zn0", "ycor", "y")
+    vals = dict(zip(names, np.random.default_rng(5).uniform(0.5, 2, (5, n))))
+    v = {k: gpu_vec(ctx, vals[k]) for k in names}
+    out, other = shared.split("=")
+    args = [v[other if k == out else k] for k in names]
+    dn, cn = C.c_double(-1.0), C.c_double(-1.0)
+    assert fn(*args, C.byref(dn), C.byref(cn)) == -1
+    assert (dn.value, cn.value) == (-1.0, -1.0)
+    assert all(np.array_equal(gpu_get(v[k]), vals[k]) for k in names)
+    for k in names:
+        core.N_VDestroy(v[k])
