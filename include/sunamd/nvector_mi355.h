@@ -8,9 +8,9 @@
  * :500-560) with the same roles:
  *   - every standard op, the fused LinearCombination / ScaleAddMulti /
  *     DotProdMulti and the vector-array ops are device kernels;
- *   - reductions finish on the device and hand one value back through a
- *     pinned host slot (one stream synchronisation per reduction, no
- *     per-call allocation or pointer-array copies);
+ *   - reductions hand their values back through pinned host slots (no
+ *     per-call allocation or pointer-array copies) and return as soon as the
+ *     host sees them: see "What a returned value says" below;
  *   - N_VGetArrayPointer returns a host mirror (allocated on first use),
  *     N_VGetDeviceArrayPointer the HBM array; the mirror is synchronised only
  *     by N_VCopyToDevice_Mi355 / N_VCopyFromDevice_Mi355.
@@ -18,6 +18,22 @@
  * Elementwise ops round exactly like the reference serial vector (same
  * formula per element, no fused multiply-add); reductions sum in a fixed
  * tree order, so they are deterministic but not bit-equal to a sequential sum.
+ *
+ * What a returned value says.  Reductions, the Gram-Schmidt step and CVODE's
+ * fused passes that return a norm do not synchronise the stream (a few return
+ * through a synchronisation all the same: every 32nd result, one that takes
+ * longer than 2 ms, N_VInvTest, N_VConstrMask and N_VMinQuotient).  When one
+ * of them returns,
+ *   - its values are final, and the ops issued on the stream before it have run;
+ *   - the stream need not be idle: vectors that the call itself writes
+ *     (cvNewtonUpdate_fused_Mi355: ycor and y; cvEwtSetSSNorm_fused_Mi355:
+ *     tempv and weight) may still be on their way;
+ *   - a failure on the stream may be reported only by the next call that
+ *     synchronises it, up to 32 results later.
+ * Work that uses the vectors belongs on their stream (N_VGetStream_Mi355), or
+ * after N_VSynchronize_Mi355, a stream synchronisation or an event recorded on
+ * it; a norm is not such a point for a buffer given to N_VMake_Mi355 that the
+ * host or another stream reads.  The copies to host arrays below synchronise.
  * ---------------------------------------------------------------------------*/
 #ifndef SUNAMD_NVECTOR_MI355_H
 #define SUNAMD_NVECTOR_MI355_H
@@ -71,7 +87,8 @@ SUNErrCode N_VSetReductionOrder_Mi355(N_Vector v, int order);
 /* HIP failures: ops that return SUNErrCode return SUN_ERR_EXT_FAIL, and the
    first failure on a vector's execution context (its stream) is also kept
    there, because void ops (N_VLinearSum, ...) cannot return it: after one,
-   reductions return NaN until it is read.  Returns that hipError_t code (0:
+   reductions return NaN until it is read (a failure while kernels run is
+   noticed when the stream is next synchronised, see above).  Returns that hipError_t code (0:
    none) and clears it; -1 for a vector that is not an MI355X vector.  (The
    reference reports through SUNContext's last error; this library never
    writes into the SUNContext, whose layout belongs to the linked core.) */
@@ -81,9 +98,11 @@ int N_VGetHipError_Mi355(N_Vector v);
    arguments, coefficients and reorthogonalisation rule
    (include/sundials/sundials_iterative.h:231-233): the k projections and
    ||v_k||^2 are summed into device memory, the update v_k -= sum h_i v_i
-   reads them there and sums the new norm in the same pass, and one
-   synchronisation returns the Hessenberg column -- 8(2k+3) bytes per element
-   and one host round trip instead of 8(2k+5) and two.  Vectors in
+   reads them there and sums the new norm in the same pass, and the Hessenberg
+   column comes back through the result slots in one host round trip instead
+   of two -- 8(2k+3) bytes per element instead of 8(2k+5) up to k = 11 (12
+   vectors per pass; each further pass reads v_k once more, and writes it once
+   more in the update).  Vectors in
    sequential reduction order take SUNClassicalGS itself.  Install with
    SUNLinSol_SPGMRSetClassicalGSFn. */
 SUNErrCode SUNAMD_ClassicalGS_Mi355(N_Vector* v, sunrealtype** h, int k, int p,

@@ -979,7 +979,9 @@ static void mi_compare(sunrealtype c, N_Vector x, N_Vector z)
 // stream synchronisation adds its own wake-up.  A slot that does not change
 // within SLOT_WAIT_S -- a kernel that takes longer, an error, a launch inside a
 // stream capture -- is left to hipStreamSynchronize, which also reports the
-// error.  Everything earlier on the stream is complete when the slot changes.
+// error.  Everything earlier on the stream is complete when the slot changes;
+// vectors that the publishing kernel itself stores (k_newton_update,
+// k_ewt_norm) need not be, nor need the stream be idle.
 static constexpr unsigned long long SLOT_EMPTY = 0x7ff4a3d5c2e1b709ULL;
 static constexpr double SLOT_WAIT_S            = 2e-3;
 // Every so many results the stream is synchronised all the same: the runtime
@@ -1797,8 +1799,8 @@ static bool gs_buffers(Mi355Exec* ex)
 
 // Same arguments, coefficients and reorthogonalisation rule as SUNClassicalGS;
 // the projections are computed into device memory, the update reads them
-// there and sums the new norm in the same pass, so one synchronisation
-// returns the Hessenberg column and both norms.  Vectors in sequential
+// there and sums the new norm in the same pass, so one round trip through the
+// result slots returns the Hessenberg column and both norms.  Vectors in sequential
 // reduction order, or more than GS_MAX basis vectors, take SUNClassicalGS.
 extern "C" SUNErrCode SUNAMD_ClassicalGS_Mi355(N_Vector* v, sunrealtype** h, int k, int p,
                                                sunrealtype* new_vk_norm, sunrealtype* stemp,
