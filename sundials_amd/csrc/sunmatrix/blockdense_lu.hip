@@ -288,9 +288,21 @@ static bool launch_getrf(int m, const double* A, T* F, int* piv, long nblocks,
   return true;
 }
 
-// The sizes compiled with m constant factor c*src + I in one pass (SRC_SCALED,
-// or SRC_SAVE with src also copied to save); false for other sizes, which take
-// the separate copy / scale / factor calls.
+// The sizes compiled with m constant have the one-pass setup and solve; the
+// others take the separate calls.
+static bool lu_one_pass(int m, int precision)
+{
+  if (precision == SUNAMD_LU_FP32)
+  {
+    const LuLaunch<float>* L = lu_launch<float>(m);
+    return L && L->getrf_scaled;
+  }
+  const LuLaunch<double>* L = lu_launch<double>(m);
+  return L && L->getrf_scaled;
+}
+
+// Factors c*src + I in one pass (SRC_SCALED, or SRC_SAVE with src also copied
+// to save); false where lu_one_pass is.
 template <typename T>
 static bool launch_getrf_scaled(int m, bool save_src, const double* src, double c, double* save,
                                 double* scaled, T* F, int* piv, long nblocks,
@@ -740,25 +752,24 @@ extern "C" int SUNLinSol_Mi355BlockLUSetupScaled(SUNLinearSolver S, SUNMatrix A,
     return SUN_ERR_ARG_INCOMPATIBLE;
   }
   const int m = (int)lc->m;
-  if (m > 10 && m != 12 && m != 16 && m != 24 && m != 32 && m != 48 && m != 64)
-  {
-    return SUN_ERR_ARG_INCOMPATIBLE;
-  }
+  if (!lu_one_pass(m, lc->precision)) { return SUN_ERR_ARG_INCOMPATIBLE; }
   const double* src = save_to_J ? BM(A)->dev : BM(J)->dev;
   double* save      = save_to_J ? BM(J)->dev : nullptr;
   k_info_reset<<<1, 1, 0, lc->stream>>>(lc->dinfo);
+  bool ok;
   sunamd_prof_begin(SUNAMD_K_GETRF, lc->stream);
   if (lc->precision == SUNAMD_LU_FP32)
   {
-    launch_getrf_scaled<float>(m, save_to_J != 0, src, c, save, BM(A)->dev, lc->f32, lc->piv,
-                               (long)lc->nblocks, lc->dinfo, lc->stream);
+    ok = launch_getrf_scaled<float>(m, save_to_J != 0, src, c, save, BM(A)->dev, lc->f32, lc->piv,
+                                    (long)lc->nblocks, lc->dinfo, lc->stream);
   }
   else
   {
-    launch_getrf_scaled<double>(m, save_to_J != 0, src, c, save, nullptr, BM(A)->dev, lc->piv,
-                                (long)lc->nblocks, lc->dinfo, lc->stream);
+    ok = launch_getrf_scaled<double>(m, save_to_J != 0, src, c, save, nullptr, BM(A)->dev,
+                                     lc->piv, (long)lc->nblocks, lc->dinfo, lc->stream);
   }
   sunamd_prof_end(SUNAMD_K_GETRF, lc->stream);
+  if (!ok) { return SUN_ERR_ARG_OUTOFRANGE; }
   return lu_finish(S);
 }
 
@@ -779,7 +790,7 @@ extern "C" int SUNLinSol_Mi355BlockLUSolveScaled(SUNLinearSolver S, SUNMatrix A,
   const int m = (int)c->m;
   if (!SUNAMD_NVectorIsMi355(b) || (hipStream_t)N_VGetStream_Mi355(b) != c->stream ||
       BM(A)->nblocks != c->nblocks || BM(A)->m != c->m || BM(A)->stream != c->stream ||
-      (m > 10 && m != 12 && m != 16 && m != 24 && m != 32 && m != 48 && m != 64))
+      !lu_one_pass(m, c->precision))
   {
     return SUN_ERR_ARG_INCOMPATIBLE;
   }

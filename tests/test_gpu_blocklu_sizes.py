@@ -13,7 +13,7 @@ import pytest
 
 from sundials_amd import _lib
 from helpers import dp, gpu_get, gpu_vec
-from test_gpu_blocklu import _gpu_matrix, _gpu_matrix_values, _to_blockmajor
+from test_gpu_blocklu import _gpu_matrix, _gpu_matrix_values, _setup_run, _to_blockmajor
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +131,41 @@ def test_scale_add_i_over_several_pairs_per_thread(ctx):
     assert np.array_equal(_gpu_matrix_values(hip, M, nb, m), a)
     core.SUNMatDestroy(M)
     core.N_VDestroy(y)
+
+
+ONE_PASS = {*range(1, 11), 12, 16, 24, 32, 48, 64}  # sizes compiled with m constant
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("m", range(1, 65))
+def test_one_pass_calls_at_every_size(ctx, m, prec):
+    """The one-pass setup and solve either do the separate calls' work bit for
+    bit or decline with everything as it was: a setup that reports success has
+    factored."""
+    core, hip = _lib.core(), _lib.hip()
+    nb = 5
+    J = np.random.default_rng(m).uniform(-1, 1, (nb, m, m)) * 4.0 / m
+    ref = _setup_run(core, hip, ctx, J, prec, 0, False, -0.25)
+    y = gpu_vec(ctx, np.zeros(nb * m))
+    MA, MJ = _gpu_matrix(hip, ctx, y, np.zeros_like(J)), _gpu_matrix(hip, ctx, y, J)
+    LS = hip.SUNLinSol_Mi355BlockLU(y, MA, prec, ctx)
+    assert core.SUNLinSolInitialize(LS) == 0
+    flag = hip.SUNLinSol_Mi355BlockLUSetupScaled(LS, MA, MJ, -0.25, 0)
+    b = np.random.default_rng(5).uniform(-1, 1, nb * m)  # the right-hand side of _setup_run
+    gb = gpu_vec(ctx, b)
+    if m in ONE_PASS:
+        assert flag == 0
+        assert np.array_equal(_gpu_matrix_values(hip, MA, nb, m), ref[1])
+        assert hip.SUNLinSol_Mi355BlockLUSolveScaled(LS, MA, gb, 1.0) == 0
+        assert np.array_equal(gpu_get(gb), ref[3])
+    else:
+        incompatible = -9998
+        assert flag == incompatible
+        assert not _gpu_matrix_values(hip, MA, nb, m).any()
+        assert hip.SUNLinSol_Mi355BlockLUSolveScaled(LS, MA, gb, 1.0) == incompatible
+        assert np.array_equal(gpu_get(gb), b)
+    core.SUNLinSolFree(LS)
+    for M in (MA, MJ):
+        core.SUNMatDestroy(M)
+    for v in (y, gb):
+        core.N_VDestroy(v)
