@@ -169,3 +169,39 @@ def test_one_pass_calls_at_every_size(ctx, m, prec):
         core.SUNMatDestroy(M)
     for v in (y, gb):
         core.N_VDestroy(v)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("m", [11, 21, 33, 41, 49, 57, 63, 64])
+def test_zero_pivot_in_every_group_width(ctx, m, prec):
+    """A zero column, which stays one through the elimination, in groups of 16, 32 and
+    64 lanes with m at run time and in 64 with m constant: the first failing
+    block's column is reported, and the other blocks' factors and pivots are
+    those of the dense solver."""
+    core, hip, orc = _lib.core(), _lib.hip(), _lib.load_oracle()
+    nb, bad, col = 6, 3, m - 2
+    A = np.random.default_rng(m).uniform(-1, 1, (nb, m, m))
+    A[bad, :, col] = 0.0
+    A[bad + 1, :, m - 1] = -0.0
+    y = gpu_vec(ctx, np.zeros(nb * m))
+    M = _gpu_matrix(hip, ctx, y, A)
+    LS = hip.SUNLinSol_Mi355BlockLU(y, M, prec, ctx)
+    assert core.SUNLinSolSetup(LS, M) == 808  # SUNLS_LUFACT_FAIL
+    assert core.SUNLinSolLastFlag(LS) == bad * m + col + 1
+    piv = np.zeros(nb * m, np.int32)
+    assert hip.SUNLinSol_Mi355BlockLU_GetPivots(LS, piv.ctypes.data_as(C.POINTER(C.c_int))) == 0
+    F = _gpu_matrix_values(hip, M, nb, m).reshape(nb, m * m)
+    for k in range(nb):
+        a, p = _numpy_getrf(A[k], np.float32 if prec else np.float64)
+        upto = {bad: col, bad + 1: m - 1}.get(k, m)  # columns before the zero pivot
+        assert np.array_equal(piv.reshape(nb, m)[k][:upto], p[:upto]), k
+        if prec == 0:
+            o = _to_blockmajor(A[k:k + 1]).copy()
+            q = np.zeros(m, np.int64)
+            rc = orc.oracle_block_getrf(dp(o), m, q.ctypes.data_as(C.POINTER(C.c_int64)))
+            assert rc == {bad: col + 1, bad + 1: m}.get(k, 0)
+            if rc == 0:
+                assert np.array_equal(F[k], o), k
+    core.SUNLinSolFree(LS)
+    core.SUNMatDestroy(M)
+    core.N_VDestroy(y)
