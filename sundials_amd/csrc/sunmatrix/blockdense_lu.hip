@@ -262,8 +262,8 @@ __global__ void __launch_bounds__(64) k_getrf_mfma(const double* __restrict__ A,
 // launch dispatch over block sizes with register-resident kernels
 // ----------------------------------------------------------------------------
 // The launch tables.  Every size up to 64 has a register-row kernel: the
-// common ones with m constant, the others with m at run time in the next row
-// length of the second list.
+// common ones their own, the others with m at run time in the next row length
+// of the second list.
 #define LU_EXACT_CASE(MM) case MM: return lu_size<MM, T>();
 #define LU_ROW_CASE(MM) if (m <= MM) { return lu_row_size<MM, T>(); }
 template <typename T>
@@ -288,7 +288,7 @@ static bool launch_getrf(int m, const double* A, T* F, int* piv, long nblocks,
   return true;
 }
 
-// The sizes compiled with m constant have the one-pass setup and solve; the
+// The sizes with launches of their own have the one-pass setup and solve; the
 // others take the separate calls.
 static bool lu_one_pass(int m, int precision)
 {

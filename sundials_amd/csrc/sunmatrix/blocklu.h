@@ -7,7 +7,7 @@
 
 #include <hip/hip_runtime.h>
 
-// the launches of one block size (getrf_scaled: null where m is not constant)
+// the launches of one block size (getrf_scaled: null for the sizes between)
 template <typename T>
 struct LuLaunch
 {
@@ -19,7 +19,7 @@ struct LuLaunch
                 double scale, hipStream_t s);
 };
 
-// Sizes compiled with m constant, and the register-row lengths that serve the
+// Sizes with launches of their own, and the register-row lengths that serve the
 // sizes between them with m at run time (the smallest one >= m).  At m = 21
 // (FP32 factors, 50000 blocks) the run-time form factors in 0.10 ms and solves
 // in 0.037 ms, where the LDS kernels it replaces, one lane working through the

@@ -22,8 +22,9 @@
 //     and upper sweeps, the solved entry broadcast by lane reads or DPP and
 //     each quotient formed from the diagonal's reciprocal with two exact
 //     remainder steps (correctly rounded, like the division).
-// The common sizes are compiled with m constant; every other m up to 64 runs
-// the kernel of the next size in a short list with m at run time.
+// The common sizes up to 32 are compiled with m constant (of 48 and 64 the
+// solve is); every other m up to 64 runs the kernel of the next size in a short
+// list with m at run time.
 // -----------------------------------------------------------------------------
 #ifndef SUNAMD_BLOCKLU_DEVICE_H
 #define SUNAMD_BLOCKLU_DEVICE_H
@@ -47,14 +48,6 @@ __device__ __forceinline__ T to_t(double v)
 {
   return (T)v;
 }
-
-// zero exactly when v is +0 or -0
-__device__ __forceinline__ unsigned magnitude_word(double v)
-{
-  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
-  return ((unsigned)(u >> 32) << 1) | (unsigned)u;
-}
-__device__ __forceinline__ unsigned magnitude_word(float v) { return __float_as_uint(v) << 1; }
 
 // How k_getrf forms the matrix it factors from its source blocks A:
 //   SRC_PLAIN  the blocks themselves;
@@ -83,7 +76,8 @@ enum GetrfSource
 // (block*m + k + 1) for the first zero pivot k.  Lane r of a block's group of
 // G = pow2ceil(M) lanes holds row r; the row swaps exchange position tags
 // only, and the rows are written to their final positions at the end.
-// RT: m is m_rt <= M at run time (M = the registers of a row), otherwise M.
+// RT: m is m_rt <= M at run time (M = the registers of a row; m_rt = M in the
+// scaled forms), otherwise M.
 //
 // What bounds it (m = 32 FP64, 2^18 blocks: 4.3 GB, 0.73 ms at the copy
 // rate): first VALU issue -- 6533 instructions per wavefront, 1.68 ms, with a
@@ -95,6 +89,14 @@ enum GetrfSource
 // the first few of a filled Newton matrix) runs without tests.  With 3151
 // instructions it takes 1.48 ms and is bound by the LDS reads of the pivot
 // row (a broadcast of 16 bytes per lane occupies the LDS for 8 cycles).
+// Rows of more than 32 entries (one block per wavefront) take the pivot row
+// from its lane entry by entry, and always in the RT form: its tests between
+// the columns keep the compiler from collecting the scalars of many columns,
+// which cost registers.  With m constant and 16 entries of the pivot row in
+// scalar registers at a time, 64 x 64 FP64 blocks needed up to 256 registers
+// (one wavefront per SIMD); now 144 to 161 (three).  40000 such blocks: set-up
+// after a copy 2.55 -> 2.18 ms, one-pass set-up 3.44 -> 1.68 ms, FP32 1.21 ->
+// 1.02 ms; 48 x 48 FP64 1.47 -> 1.27 and 1.22 -> 0.93 ms.
 template <int M, typename T, int SRC = SRC_PLAIN, bool RT = false>
 __global__ void __launch_bounds__(64 * LU_WAVES) k_getrf(const double* A, T* F /* may alias A */,
                                                          int* __restrict__ piv, long nblocks,
@@ -185,51 +187,29 @@ __global__ void __launch_bounds__(64 * LU_WAVES) k_getrf(const double* A, T* F /
       const T pk   = readlane_d(a[k], pl);
       const T mult = readlane_d(rk, pl);
       if (r == k) { myp = bp; }
-      if (magnitude_word(pk) == 0 && fail == 0) { fail = k + 1; }
+      if (pk == (T)0 && fail == 0) { fail = k + 1; }
       if (win) { pos = k; }
       else if (pos == k) { pos = bp; }
-      if (valid && pos > k && fail == 0)
+      const bool up = valid && pos > k && fail == 0;
+      T l           = (T)0;
+      if (up)
       {
-        const T l = a[k] * mult;
-        a[k]      = l;
-        // the pivot row in chunks through scalar registers: the zero test is
-        // scalar work (the smallest magnitude's bits), once per chunk
-        constexpr int PC = 16;
+        l    = a[k] * mult;
+        a[k] = l;
+      }
+      // (in chunks so that columns past a run-time m are skipped)
+      constexpr int PC = 16;
 #pragma unroll
-        for (int j0 = k + 1; j0 < M; j0 += PC)
+      for (int j0 = k + 1; j0 < M; j0 += PC)
+      {
+        if (RT && j0 >= m) { continue; }
+#pragma unroll
+        for (int q = 0; q < PC; q++)
         {
-          if (RT && j0 >= m) { continue; }
-          T pj[PC];
-          unsigned least = ~0u;
-#pragma unroll
-          for (int q = 0; q < PC; q++)
+          if (j0 + q < M)
           {
-            if (j0 + q < M)
-            {
-              pj[q]              = readlane_d(a[j0 + q], pl);
-              const unsigned mag = magnitude_word(pj[q]);
-              least              = mag < least ? mag : least;
-            }
-          }
-          if (least != 0)
-          {
-#pragma unroll
-            for (int q = 0; q < PC; q++)
-            {
-              if (j0 + q < M) { a[j0 + q] = a[j0 + q] - pj[q] * l; }
-            }
-          }
-          // (two ifs, not if / else: the entries then stay in their registers)
-          if (least == 0)
-          {
-#pragma unroll
-            for (int q = 0; q < PC; q++)
-            {
-              if (j0 + q < M && magnitude_word(pj[q]) != 0)
-              {
-                a[j0 + q] = a[j0 + q] - pj[q] * l;
-              }
-            }
+            const T pj = readlane_d(a[j0 + q], pl);
+            if (up && pj != (T)0) { a[j0 + q] = a[j0 + q] - pj * l; }
           }
         }
       }
@@ -419,18 +399,18 @@ void lu_getrf(int m, const double* A, T* F, int* piv, long nblocks, unsigned lon
     <<<lu_grid(M, nblocks), 64 * LU_WAVES, 0, s>>>(A, F, piv, nblocks, info, m);
 }
 
-template <int M, typename T>
+template <int M, typename T, bool RT>
 void lu_getrf_scaled(bool save_src, const double* src, double c, double* save, double* scaled,
                      T* F, int* piv, long nblocks, unsigned long long* info, hipStream_t s)
 {
   if (save_src)
   {
-    k_getrf<M, T, SRC_SAVE><<<lu_grid(M, nblocks), 64 * LU_WAVES, 0, s>>>(
+    k_getrf<M, T, SRC_SAVE, RT><<<lu_grid(M, nblocks), 64 * LU_WAVES, 0, s>>>(
       src, F, piv, nblocks, info, M, c, save, scaled);
   }
   else
   {
-    k_getrf<M, T, SRC_SCALED><<<lu_grid(M, nblocks), 64 * LU_WAVES, 0, s>>>(
+    k_getrf<M, T, SRC_SCALED, RT><<<lu_grid(M, nblocks), 64 * LU_WAVES, 0, s>>>(
       src, F, piv, nblocks, info, M, c, save, scaled);
   }
 }
@@ -445,7 +425,8 @@ void lu_getrs(int m, const T* F, const int* piv, const double* b, double* x, lon
 template <int M, typename T>
 const LuLaunch<T>* lu_size()
 {
-  static const LuLaunch<T> L = {lu_getrf<M, T, false>, lu_getrf_scaled<M, T>,
+  constexpr bool RT          = M > 32; // rows longer than 32: see k_getrf
+  static const LuLaunch<T> L = {lu_getrf<M, T, RT>, lu_getrf_scaled<M, T, RT>,
                                 lu_getrs<M, T, false>};
   return &L;
 }
