@@ -74,7 +74,8 @@ __device__ __forceinline__ void ma_stage_tables(const int* __restrict__ idx,
 // on: its species of this lane and the rates of this lane's first two
 // reactions (R = 1.5 m needs no more; further ones are loaded where they are
 // used).  Lanes without a cell or a reaction read inside the arrays and drop
-// the value, so the loads are unconditional.
+// the value, so the loads are unconditional; a workgroup's last pass fetches
+// nothing (every workgroup would read the last cell).
 struct MaNext
 {
   double y, kf[2], kb[2];
@@ -105,8 +106,9 @@ __device__ __forceinline__ MaNext ma_fetch(const double* __restrict__ y,
 // What bounds it: LDS and VALU issue about as much as HBM (m = 32, R = 48:
 // 1280 bytes per cell; 2^18 cells in 57 us at the copy rate).  A lane's terms
 // are the same for every cell, so the first MA_TERMS of them (their rate's
-// place and sign) stay in registers instead of being read from LDS per cell:
-// 101 -> 98 us.
+// place and sign) stay in registers instead of being read from LDS per cell,
+// which pays from the second pass of a workgroup on: 2^18 cells 75 -> 66 us,
+// 30000 cells 12.4 -> 9.5 us with one round of workgroups (14.1 with four).
 constexpr int MA_TERMS = 12;
 
 __global__ void __launch_bounds__(64) k_ma_rhs(const double* __restrict__ y,
@@ -154,7 +156,7 @@ __global__ void __launch_bounds__(64) k_ma_rhs(const double* __restrict__ y,
     const MaNext nc = nx;
     if (live && i < m) { ys[i] = nc.y; }
     wave_sync();
-    nx = ma_fetch(y, kf, kb, cell + step, ncells, i, m, G, R);
+    if (c0 + step < ncells) { nx = ma_fetch(y, kf, kb, cell + step, ncells, i, m, G, R); }
     if (live)
     {
 #pragma unroll
@@ -227,7 +229,7 @@ struct MaTerm
 // 0.41 ms at the copy rate) against the chain of LDS updates of a row.  So the
 // next cell's operands are fetched meanwhile, a term's operands are read while
 // the one before it updates the row, and the block is cleared as it is
-// written out (in pairs of doubles where m*m is even): 0.58 -> 0.43 ms.
+// written out (in pairs of doubles where m*m is even): 2^18 cells 560 -> 450 us.
 template <bool PAIRS>
 __global__ void __launch_bounds__(64) k_ma_jac(const double* __restrict__ y,
                                                double* __restrict__ J,
@@ -296,7 +298,7 @@ __global__ void __launch_bounds__(64) k_ma_jac(const double* __restrict__ y,
       }
     }
     wave_sync();
-    nx = ma_fetch(y, kf, kb, cell + step, ncells, i, m, G, R);
+    if (c0 + step < ncells) { nx = ma_fetch(y, kf, kb, cell + step, ncells, i, m, G, R); }
     if (live && e0 < e1)
     {
       // row i: the terms in which species i is a target, each adding the
@@ -336,6 +338,85 @@ __global__ void __launch_bounds__(64) k_ma_jac(const double* __restrict__ y,
           Jl[e] = 0.0;
         }
       }
+    }
+    wave_sync();
+  }
+}
+
+// The same for small blocks (m < 16), cell after cell: their few terms and
+// bytes leave nothing for the operands fetched ahead to hide, and the form
+// above takes up to 8 % longer (500000 cells, four rounds: m = 5, R = 8 84
+// against 81 us; m = 11, R = 16 212 against 208; but m = 16, R = 24 301 against
+// 359).
+__global__ void __launch_bounds__(64) k_ma_jac_small(const double* __restrict__ y,
+                                               double* __restrict__ J,
+                                               const int* __restrict__ idx,
+                                               const int* __restrict__ soff,
+                                               const int* __restrict__ sent,
+                                               const double* __restrict__ kf,
+                                               const double* __restrict__ kb, int m, int G,
+                                               int R, long ncells)
+{
+  using sunamd_lane::wave_sync;
+  extern __shared__ __align__(16) double sj[];
+  const int gpw   = 64 / G;
+  const int mm    = m * m;
+  const long per  = (long)((mm + m + 2 * R + 1) & ~1);
+  const int grp   = threadIdx.x / G;
+  const int i     = threadIdx.x % G;
+  double* Jl      = sj + grp * per;
+  double* ys      = Jl + mm;
+  double* rk      = ys + m;
+  int* s_idx      = (int*)(sj + gpw * per);
+  int* s_sent     = s_idx + 4 * R;
+  int* s_soff     = s_sent + 4 * R;
+  ma_stage_tables(idx, soff, sent, s_idx, s_soff, s_sent, m, R);
+  __syncthreads();
+  const int e0    = (i < m) ? s_soff[i] : 0;
+  const int e1    = (i < m) ? s_soff[i + 1] : 0;
+  const int4* ix4 = (const int4*)s_idx;
+  for (long c0 = (long)blockIdx.x * gpw; c0 < ncells; c0 += (long)gridDim.x * gpw)
+  {
+    const long cell = c0 + grp;
+    const bool live = cell < ncells;
+    if (live)
+    {
+      for (int e = i; e < mm; e += G) { Jl[e] = 0.0; }
+      if (i < m) { ys[i] = y[cell * m + i]; }
+      for (int r = i; r < R; r += G)
+      {
+        rk[r]     = kf[cell * R + r];
+        rk[R + r] = kb[cell * R + r];
+      }
+    }
+    wave_sync();
+    if (live && i < m)
+    {
+      // row i: the terms in which species i is a target, each adding the
+      // reaction's partial derivatives to the columns of its four species
+      for (int e = e0; e < e1; e++)
+      {
+        const int code  = s_sent[e];
+        const int r     = code >> 2;
+        const bool loss = (code & 3) < 2;
+        const int4 ix   = ix4[r];
+        const double kfv = rk[r], kbv = rk[R + r];
+        const int col[4]   = {ix.x, ix.y, ix.z, ix.w};
+        const double dw[4] = {kfv * ys[ix.y], kfv * ys[ix.x], -(kbv * ys[ix.w]),
+                              -(kbv * ys[ix.z])};
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+          const int a = col[q] * m + i;
+          Jl[a]       = loss ? (Jl[a] - dw[q]) : (Jl[a] + dw[q]);
+        }
+      }
+    }
+    wave_sync();
+    if (live)
+    {
+      double* Jc = J + cell * (long)mm;
+      for (int e = i; e < mm; e += G) { Jc[e] = Jl[e]; }
     }
     wave_sync();
   }
@@ -436,10 +517,7 @@ extern "C" void SUNAMD_MassActionDevFree(SUNAMD_MassActionDev* d)
 }
 
 // workgroups for a grid-stride launch: enough to fill every CU `rounds` times
-// at the kernel's occupancy, no more than the cells need.  The Jacobian's take
-// one round (m = 32, 2^18 cells: 431 us, 466 with two, 478 with eight -- fewer
-// table stagings, and a long run of prefetched cells each), the right-hand
-// side's four (98 us, 103 with one: its short passes leave wavefronts uneven).
+// at the kernel's occupancy, no more than the cells need
 template <typename K>
 static unsigned ma_grid(K kern, size_t shm, long ncells, int gpw, int rounds)
 {
@@ -472,7 +550,10 @@ extern "C" int SUNAMD_MassActionRhsDevArrays(SUNAMD_MassActionDev* d, const doub
   const int gpw = 64 / G;
   const size_t shm = ma_rhs_lds(d->m, d->R);
   if (d->ncells < 1) { return 0; }
-  if (d->rhs_grid == 0) { d->rhs_grid = ma_grid(k_ma_rhs, shm, d->ncells, gpw, 4); }
+  // one round: fewer table stagings and term lists, a longer run of prefetched
+  // cells each (with four, 120000 cells of m = 5, R = 8 took 11.5 us, with one
+  // 8.0; cell after cell without either it was 9.3)
+  if (d->rhs_grid == 0) { d->rhs_grid = ma_grid(k_ma_rhs, shm, d->ncells, gpw, 1); }
   const unsigned g = d->rhs_grid;
   sunamd_prof_begin(SUNAMD_K_RHS, d->stream);
   k_ma_rhs<<<g, 64, shm, d->stream>>>(dy, df, d->idx, d->soff, d->sent, d->kf, d->kb, d->m, G,
@@ -490,9 +571,20 @@ extern "C" int SUNAMD_MassActionJacDevArrays(SUNAMD_MassActionDev* d, const doub
   const size_t shm = ma_jac_lds(d->m, d->R);
   if (d->ncells < 1) { return 0; }
   // blocks of an even number of entries start on 16 bytes if the array does
-  const bool pairs = (d->m * d->m) % 2 == 0 && ((uintptr_t)dJ & 15u) == 0;
-  auto kern        = pairs ? k_ma_jac<true> : k_ma_jac<false>;
-  if (d->jac_grid == 0) { d->jac_grid = ma_grid(k_ma_jac<true>, shm, d->ncells, gpw, 1); }
+  const int mm     = d->m * d->m;
+  const bool pairs = mm % 2 == 0 && ((uintptr_t)dJ & 15u) == 0;
+  const bool small = d->m < 16;
+  auto kern        = small ? k_ma_jac_small : pairs ? k_ma_jac<true> : k_ma_jac<false>;
+  if (d->jac_grid == 0)
+  {
+    // one round where writing the block outweighs the 16R updates of its
+    // entries, four where the updates do and the wavefronts end unevenly
+    // (120000 cells, one against four: m = 32, R = 48 209 / 223 us, R = 96
+    // 487 / 362; m = 24, R = 36 188 / 161; 30000 cells of 64, R = 96 208 / 221)
+    const int rounds = (mm >= 1024 && mm >= 16 * d->R) ? 1 : 4;
+    d->jac_grid      = small ? ma_grid(k_ma_jac_small, shm, d->ncells, gpw, rounds)
+                             : ma_grid(k_ma_jac<true>, shm, d->ncells, gpw, rounds);
+  }
   const unsigned g = d->jac_grid;
   kern<<<g, 64, shm, d->stream>>>(dy, dJ, d->idx, d->soff, d->sent, d->kf, d->kb, d->m, G, d->R,
                                   d->ncells);
