@@ -103,9 +103,9 @@ __device__ __forceinline__ double lsum(double a, double x, double b, double y)
   return (a * x) + (b * y);
 }
 
-// lsum with b = 1, whose three forms give the same bits: 1*y is y, and for
+// lsum with b = 1, whose three forms give the same value: 1*y is y, and for
 // a = 1 the sum x + y, for a = -1 the difference y - x is what each rounds
-// (they differ only in the sign of an exact zero for a = -1)
+// (the same bits, but for the sign of an exact zero where a = -1)
 __device__ __forceinline__ double lsum1(double a, double x, double y) { return (a * x) + y; }
 
 __device__ __forceinline__ double sqrt0(double v) { return (v <= 0.0) ? 0.0 : sqrt(v); }
@@ -513,15 +513,18 @@ __device__ __forceinline__ void g_diagonal(const Grp<M, T>& g, Sys<M, T>& S)
 
 // ---- LU of the group's matrix (rows in lanes, implicit pivoting) ---------
 // The FP64 form follows the dense GETRF operation by operation; as in the
-// block solver's k_getrf, the pivot search exchanges one word per level, the
-// pivot's reciprocal is formed beside it and (groups of up to 32 lanes) the
-// zero test is made once per column.
-// What bounds the integrator: the FP32 form's VALU issue (three wavefronts per
-// SIMD keep it 91 % busy, 3000 vector instructions per step), the FP64 form's
-// chains of dependent operations and LDS round trips (two per SIMD).  This
-// factorisation, the solves below, lsum1, the operands read ahead in g_rhs and
-// g_newton_matrix and the constant lane masks together took the uneven batch
-// of 65536 systems from 181 to 165 ms (FP64) and from 85.7 to 81.4 ms (FP32).
+// block solver's k_getrf, the pivot search exchanges one word per level and, in
+// groups of up to 32 lanes, the pivot's reciprocal is formed beside it and the
+// zero test is made once per column.  One system per wavefront (G = 64): the
+// pivot row is read from its lane's registers, and the reciprocal is formed
+// from the pivot after the search -- every lane's own beside it made rows of 48
+// doubles spill 347 registers instead of 86 at two wavefronts per SIMD (512
+// systems of 48: 17.5 -> 15.2 ms; FP32, with the pivot row no longer through
+// LDS, 9.1 -> 8.4 ms).
+// What bounds the integrator (a bucket alone, two wavefronts per SIMD): chains
+// of dependent operations and LDS round trips.  The vector units are busy 62 to
+// 67 % of the time for FP32 factors of m >= 8 and 41 to 65 % for FP64; a
+// wavefront waits for an operand 31 to 41 % of its time.
 template <int M, typename T>
 __device__ __forceinline__ int g_getrf(const Grp<M, T>& g, Sys<M, T>& S)
 {
@@ -546,33 +549,46 @@ __device__ __forceinline__ int g_getrf(const Grp<M, T>& g, Sys<M, T>& S)
       else if (pos == bp) { pos = k; }
       // single precision: multiplier 0 on the rows not updated, fused
       // multiply-add, no zero test
-      gsync();
-      if (g.valid && pos == k)
+      if constexpr (G == 64)
       {
+        const int pl  = __builtin_amdgcn_readfirstlane(
+                         __ffsll((long long)sunamd_lane::ballot(g.valid && pos == k)) - 1) & 63;
+        const bool up = g.valid && pos > k && fail == 0;
+        const T pk    = readlane_d(S.lu[k], pl);
+        const T l     = up ? S.lu[k] * ((T)1 / pk) : (T)0;
+        if (up) { S.lu[k] = l; }
 #pragma unroll
-        for (int j = k; j < M; j++) { g.prow[j] = S.lu[j]; }
+        for (int j = k + 1; j < M; j++) { S.lu[j] = __builtin_fmaf(-readlane_d(S.lu[j], pl), l, S.lu[j]); }
       }
-      gsync();
-      const bool up = g.valid && pos > k && fail == 0;
-      const T l     = up ? S.lu[k] * ((T)1 / g.prow[k]) : (T)0;
-      if (up) { S.lu[k] = l; }
+      else
+      {
+        gsync();
+        if (g.valid && pos == k)
+        {
 #pragma unroll
-      for (int j = k + 1; j < M; j++) { S.lu[j] = __builtin_fmaf(-g.prow[j], l, S.lu[j]); }
+          for (int j = k; j < M; j++) { g.prow[j] = S.lu[j]; }
+        }
+        gsync();
+        const bool up = g.valid && pos > k && fail == 0;
+        const T l     = up ? S.lu[k] * ((T)1 / g.prow[k]) : (T)0;
+        if (up) { S.lu[k] = l; }
+#pragma unroll
+        for (int j = k + 1; j < M; j++) { S.lu[j] = __builtin_fmaf(-g.prow[j], l, S.lu[j]); }
+      }
     }
     else
     {
-      const T rk     = (T)1 / S.lu[k];
+      const T rk     = (G == 64) ? (T)0 : (T)1 / S.lu[k]; // (the pivot row's, for G < 64)
       const bool win = sunamd_lane::g_pivot<G>(S.lu[k], g.valid && pos >= k, pos, k, g.base);
       if constexpr (G == 64)
       {
         // one system per wavefront: the pivot row's lane is wavefront-uniform,
-        // its entries are read straight from that lane's registers (rows of
-        // 48 and 64 doubles leave none for a pivot row on its way from LDS)
+        // its entries are read straight from that lane's registers
         const int pl = __builtin_amdgcn_readfirstlane(
                          __ffsll((long long)sunamd_lane::ballot(win)) - 1) & 63;
         const int bp = __builtin_amdgcn_readlane(pos, pl);
         const T pk   = readlane_d(S.lu[k], pl);
-        const T mult = readlane_d(rk, pl);
+        const T mult = (T)1 / pk;
         if (pk == (T)0 && fail == 0) { fail = k + 1; }
         if (win) { pos = k; }
         else if (pos == k) { pos = bp; }
