@@ -708,8 +708,9 @@ extern "C" int SUNAMD_BatchedBDFSolveBucketNoAlloc(int m, int R, int64_t ncells,
   const long want = (A.ncells + gpw - 1) / gpw;
   const long cap  = (long)cus * 16;
   const int grid  = (int)(want < cap ? want : cap);
-  // two wavefronts per SIMD: the register budget the autotuner picks for
-  // every bucket of the benchmark batch
+  // a budget of two wavefronts per SIMD: the FP64 kernels' fastest, and within
+  // a few per cent of the FP32 kernels' (the benchmark's calibration picks one
+  // or two for them, by bucket)
   switch (m)
   {
 #define BDF_CASE(MM)                                                                     \

@@ -1,8 +1,8 @@
 // -----------------------------------------------------------------------------
 // lane_ops.h -- cross-lane primitives of the register-row LU kernels (the
 // block solver's and the batched integrator's): DPP row permutations, lane
-// reads, and the pivot search of a group of G lanes as a (value, row)
-// maximum with ties to the smaller row.
+// reads and broadcasts, constant lane masks, the pivot search of a group of G
+// lanes on one word per exchange, and quotients from an early reciprocal.
 // -----------------------------------------------------------------------------
 #ifndef SUNAMD_LANE_OPS_H
 #define SUNAMD_LANE_OPS_H

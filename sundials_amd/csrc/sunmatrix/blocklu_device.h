@@ -19,9 +19,10 @@
 //   * rows are written back to their final physical position, so the stored
 //     factors and the pivot vector are those of the reference;
 //   * GETRS permutes b through the pivot sequence, then runs the unit-lower
-//     and upper sweeps, the solved entry broadcast by lane reads or DPP and
-//     each quotient formed from the diagonal's reciprocal with two exact
-//     remainder steps (correctly rounded, like the division).
+//     and upper sweeps, the solved entry broadcast by a lane read (groups of
+//     64), an LDS shuffle (32) or DPP (up to 16), and each quotient formed
+//     from the diagonal's reciprocal with two exact remainder steps
+//     (correctly rounded, like the division).
 // The common sizes up to 32 are compiled with m constant (of 48 and 64 the
 // solve is); every other m up to 64 runs the kernel of the next size in a short
 // list with m at run time.
@@ -87,8 +88,10 @@ enum GetrfSource
 // zero test is made once per column: each lane looks at one entry of the pivot
 // row, and a column whose pivot row has no zero right of the pivot (all but
 // the first few of a filled Newton matrix) runs without tests.  With 3151
-// instructions it takes 1.48 ms and is bound by the LDS reads of the pivot
-// row (a broadcast of 16 bytes per lane occupies the LDS for 8 cycles).
+// instructions it takes 1.48 ms, and no unit is full: the LDS data path is busy
+// 59 % of the time and the vector units 53 %; a wavefront (3.9 per SIMD) waits
+// for an operand 30 % of its time -- the search, publish and read chain of a
+// column -- and 41 % for its turn to issue, mostly for an LDS instruction.
 // Rows of more than 32 entries (one block per wavefront) take the pivot row
 // from its lane entry by entry, and always in the RT form: its tests between
 // the columns keep the compiler from collecting the scalars of many columns,
