@@ -571,7 +571,7 @@ FAM_GETRS, FAM_GETRF, FAM_LINSUM, FAM_WRMS, FAM_ADR_FE, FAM_SCALE = 0, 1, 2, 3, 
 MEASURED_STREAM_TRAFFIC = {
     ("kinsol-newton", "N_VLinearSum"): 151.0e6,
     ("kinsol-newton", "N_VScale"): 100.7e6,
-    ("kinsol-newton", "k_getrs (6x6 blocks)"): 436.3e6,
+    ("kinsol-newton", "k_getrs (6x6 blocks)"): 427.9e6,
     ("kinsol-newton", "k_getrf (6x6 blocks)"): 629.2e6,
     ("kinsol", "N_VLinearSum"): 151.0e6,
     ("kinsol", "N_VScale"): 100.7e6,
@@ -587,7 +587,7 @@ def stream_traffic(workload, kernel, n):
 
 # the kernel source the MEASURED_TRAFFIC figures were taken at (first 16 hex digits of the
 # SHA-256 of bdf_device.h followed by bdf_args.h); a changed kernel reports traffic null
-MEASURED_TRAFFIC_SOURCE = "99e45596109fa425"
+MEASURED_TRAFFIC_SOURCE = "6a17b4838a10cd91"
 
 
 def batched_kernel_source_hash():
@@ -600,26 +600,33 @@ def batched_kernel_source_hash():
     return h.hexdigest()[:16]
 
 
-# HBM bytes per launch of the FP32-LU kernels at three wavefronts per SIMD (8 workgroups
-# per CU) and at two (32 workgroups per CU), rocprofv3 --pmc FETCH_SIZE x 2.000 + WRITE_SIZE
+# HBM bytes per launch of the FP32-LU kernels at budgets of one and two wavefronts per SIMD
+# (16 workgroups per CU) and three (8), rocprofv3 --pmc FETCH_SIZE x 2.000 + WRITE_SIZE
 # x 1.000 (the factors a plain 256 MiB copy gives) on the 65,536-system batch; at three
-# wavefronts almost all of it is register-spill stores, at two it is close to the
+# wavefronts almost all of it is register-spill stores, at one and two it is close to the
 # algorithmic traffic (states, rate constants, counters: ~10-20 MB per launch)
 MEASURED_TRAFFIC = {
-"k_batched_bdf<4, float, 3, false>": 19.3e6,
-    "k_batched_bdf<8, float, 3, false>": 34.1e6,
-    "k_batched_bdf<16, float, 3, false>": 343.3e6,
-    "k_batched_bdf<24, float, 3, false>": 147.0e6,
-    "k_batched_bdf<32, float, 3, false>": 1135.8e6,
-    "k_batched_bdf<48, float, 3, false>": 3379.8e6,
-    "k_batched_bdf<64, float, 3, false>": 6312.7e6,
-    "k_batched_bdf<4, float, 2, false>": 8.5e6,
+    "k_batched_bdf<4, float, 1, false>": 8.6e6,
+    "k_batched_bdf<8, float, 1, false>": 11.9e6,
+    "k_batched_bdf<16, float, 1, false>": 12.6e6,
+    "k_batched_bdf<24, float, 1, false>": 11.0e6,
+    "k_batched_bdf<32, float, 1, false>": 12.5e6,
+    "k_batched_bdf<48, float, 1, false>": 10.8e6,
+    "k_batched_bdf<64, float, 1, false>": 12.4e6,
+    "k_batched_bdf<4, float, 2, false>": 8.6e6,
     "k_batched_bdf<8, float, 2, false>": 11.9e6,
     "k_batched_bdf<16, float, 2, false>": 12.6e6,
-    "k_batched_bdf<24, float, 2, false>": 11.1e6,
-    "k_batched_bdf<32, float, 2, false>": 15.7e6,
-    "k_batched_bdf<48, float, 2, false>": 15.1e6,
-    "k_batched_bdf<64, float, 2, false>": 16.2e6,
+    "k_batched_bdf<24, float, 2, false>": 11.0e6,
+    "k_batched_bdf<32, float, 2, false>": 12.5e6,
+    "k_batched_bdf<48, float, 2, false>": 10.8e6,
+    "k_batched_bdf<64, float, 2, false>": 14.2e6,
+    "k_batched_bdf<4, float, 3, false>": 20.7e6,
+    "k_batched_bdf<8, float, 3, false>": 40.8e6,
+    "k_batched_bdf<16, float, 3, false>": 1734.4e6,
+    "k_batched_bdf<24, float, 3, false>": 70.1e6,
+    "k_batched_bdf<32, float, 3, false>": 2857.1e6,
+    "k_batched_bdf<48, float, 3, false>": 2209.9e6,
+    "k_batched_bdf<64, float, 3, false>": 8639.0e6,
 }
 
 
