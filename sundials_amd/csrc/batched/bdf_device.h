@@ -513,14 +513,15 @@ __device__ __forceinline__ void g_diagonal(const Grp<M, T>& g, Sys<M, T>& S)
 
 // ---- LU of the group's matrix (rows in lanes, implicit pivoting) ---------
 // The FP64 form follows the dense GETRF operation by operation; as in the
-// block solver's k_getrf, the pivot search exchanges one word per level and, in
-// groups of up to 32 lanes, the pivot's reciprocal is formed beside it and the
+// block solver's k_getrf, the pivot search exchanges one word per level, the
+// pivot's reciprocal is formed beside it and, in groups of up to 32 lanes, the
 // zero test is made once per column.  One system per wavefront (G = 64): the
-// pivot row is read from its lane's registers, and the reciprocal is formed
-// from the pivot after the search -- every lane's own beside it made rows of 48
-// doubles spill 347 registers instead of 86 at two wavefronts per SIMD (512
-// systems of 48: 17.5 -> 15.2 ms; FP32, with the pivot row no longer through
-// LDS, 9.1 -> 8.4 ms).
+// pivot row is read from its lane's registers.  Rows of 48 doubles form the
+// reciprocal from the pivot after the search: every lane's own beside it made
+// them spill 347 registers instead of 86 at two wavefronts per SIMD (512 systems:
+// 17.5 -> 15.2 ms; FP32, with the pivot row no longer through LDS, 9.1 -> 8.4).
+// Rows of 64 spill as much either way, and keep it beside the search (coupled,
+// 2048 cells: 390 against 420 ms).
 // What bounds the integrator (a bucket alone, two wavefronts per SIMD): chains
 // of dependent operations and LDS round trips.  The vector units are busy 62 to
 // 67 % of the time for FP32 factors of m >= 8 and 41 to 65 % for FP64; a
@@ -578,8 +579,9 @@ __device__ __forceinline__ int g_getrf(const Grp<M, T>& g, Sys<M, T>& S)
     }
     else
     {
-      const T rk     = (G == 64) ? (T)0 : (T)1 / S.lu[k]; // (the pivot row's, for G < 64)
-      const bool win = sunamd_lane::g_pivot<G>(S.lu[k], g.valid && pos >= k, pos, k, g.base);
+      constexpr bool kLate = (G == 64 && M < 64); // reciprocal after the search
+      const T rk           = kLate ? (T)0 : (T)1 / S.lu[k];
+      const bool win       = sunamd_lane::g_pivot<G>(S.lu[k], g.valid && pos >= k, pos, k, g.base);
       if constexpr (G == 64)
       {
         // one system per wavefront: the pivot row's lane is wavefront-uniform,
@@ -588,7 +590,7 @@ __device__ __forceinline__ int g_getrf(const Grp<M, T>& g, Sys<M, T>& S)
                          __ffsll((long long)sunamd_lane::ballot(win)) - 1) & 63;
         const int bp = __builtin_amdgcn_readlane(pos, pl);
         const T pk   = readlane_d(S.lu[k], pl);
-        const T mult = (T)1 / pk;
+        const T mult = kLate ? (T)1 / pk : readlane_d(rk, pl);
         if (pk == (T)0 && fail == 0) { fail = k + 1; }
         if (win) { pos = k; }
         else if (pos == k) { pos = bp; }
