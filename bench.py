@@ -587,7 +587,7 @@ def stream_traffic(workload, kernel, n):
 
 # the kernel source the MEASURED_TRAFFIC figures were taken at (first 16 hex digits of the
 # SHA-256 of bdf_device.h followed by bdf_args.h); a changed kernel reports traffic null
-MEASURED_TRAFFIC_SOURCE = "6a17b4838a10cd91"
+MEASURED_TRAFFIC_SOURCE = "ffbb2b63052443b4"
 
 
 def batched_kernel_source_hash():
@@ -609,24 +609,24 @@ MEASURED_TRAFFIC = {
     "k_batched_bdf<4, float, 1, false>": 8.6e6,
     "k_batched_bdf<8, float, 1, false>": 11.9e6,
     "k_batched_bdf<16, float, 1, false>": 12.6e6,
-    "k_batched_bdf<24, float, 1, false>": 11.0e6,
+    "k_batched_bdf<24, float, 1, false>": 11.1e6,
     "k_batched_bdf<32, float, 1, false>": 12.5e6,
     "k_batched_bdf<48, float, 1, false>": 10.8e6,
-    "k_batched_bdf<64, float, 1, false>": 12.4e6,
+    "k_batched_bdf<64, float, 1, false>": 14.2e6,
     "k_batched_bdf<4, float, 2, false>": 8.6e6,
     "k_batched_bdf<8, float, 2, false>": 11.9e6,
     "k_batched_bdf<16, float, 2, false>": 12.6e6,
     "k_batched_bdf<24, float, 2, false>": 11.0e6,
     "k_batched_bdf<32, float, 2, false>": 12.5e6,
     "k_batched_bdf<48, float, 2, false>": 10.8e6,
-    "k_batched_bdf<64, float, 2, false>": 14.2e6,
+    "k_batched_bdf<64, float, 2, false>": 12.4e6,
     "k_batched_bdf<4, float, 3, false>": 20.7e6,
-    "k_batched_bdf<8, float, 3, false>": 40.8e6,
-    "k_batched_bdf<16, float, 3, false>": 1734.4e6,
-    "k_batched_bdf<24, float, 3, false>": 70.1e6,
-    "k_batched_bdf<32, float, 3, false>": 2857.1e6,
-    "k_batched_bdf<48, float, 3, false>": 2209.9e6,
-    "k_batched_bdf<64, float, 3, false>": 8639.0e6,
+    "k_batched_bdf<8, float, 3, false>": 40.6e6,
+    "k_batched_bdf<16, float, 3, false>": 1757.4e6,
+    "k_batched_bdf<24, float, 3, false>": 70.4e6,
+    "k_batched_bdf<32, float, 3, false>": 2788.5e6,
+    "k_batched_bdf<48, float, 3, false>": 2223.1e6,
+    "k_batched_bdf<64, float, 3, false>": 6246.7e6,
 }
 
 
